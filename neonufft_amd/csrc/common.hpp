@@ -122,7 +122,7 @@ struct alignas(2 * sizeof(T)) Cplx {
 // order). x[d] is the Horner argument in [0,1): x = ceil(xi - ns/2) - (xi - ns/2)
 // for the fine-grid coordinate xi = u * n, computed in FP64 and rounded once.
 // `cell` packs, per dimension, the first kernel cell relative to the bin's
-// tile origin (bin origin - floor(ns/2)); the range is [0, bin_size].
+// tile origin (bin origin - floor(ns/2)); the range is [0, bin_size).
 // ---------------------------------------------------------------------------
 template <typename T, int DIM>
 struct PointRec;
@@ -201,7 +201,7 @@ struct BinGeom {
   int n[3];      // grid size per dim (1 for unused dims)
   int bin[3];    // bin edge per dim
   int nbins[3];  // number of bins per dim
-  int tile[3];   // LDS tile pitch per dim = bin + ns (1 for unused dims)
+  int tile[3];   // LDS tile pitch per dim = bin + ns - 1 (1 for unused dims)
 };
 
 // How raw coordinates map to the grid: v = (x - offset) * scale, then the

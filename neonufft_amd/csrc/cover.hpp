@@ -12,7 +12,7 @@
 namespace nnf {
 
 // The tile of bin b along one dimension starts ns/2 cells before the bin and
-// spans min(bin, n - b * bin) + ns cells, periodically. Cell c is covered by
+// spans min(bin, n - b * bin) + ns - 1 cells, periodically. Cell c is covered by
 // bin b at every tile position l < extent with l = (c - start) mod n + k n.
 // Only bins within ceil(ns / bin) + 1 of c's own bin can cover it, so those
 // are the candidates (all bins when there are few).
@@ -45,7 +45,7 @@ inline CoverHost build_cover(int dim, const BinGeom& g, int ns) {
       }
       for (int b : cand) {
         const long long org = static_cast<long long>(b) * B - half;
-        const int ext = std::min(B, n - b * B) + ns;
+        const int ext = std::min(B, n - b * B) + ns - 1;
         long long l = ((c - org) % n + n) % n;
         for (; l < ext; l += n) h.entry[d].push_back(make_int2(b, static_cast<int>(l)));
       }

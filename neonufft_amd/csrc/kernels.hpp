@@ -64,7 +64,7 @@ template <typename T>
 void launch_minmax(const T* x, std::size_t m, double* partial, hipStream_t stream);
 
 // ---- spread_interp.hip: ES spreading / interpolation on binned points -----
-// Cells of one subgrid tile (bin + ns halo), the pitch of every stored tile.
+// Cells of one subgrid tile (bin + halo of ns - 1), the pitch of every stored tile.
 __host__ __device__ inline std::size_t tile_cells(const BinGeom& g) {
   return static_cast<std::size_t>(g.tile[0]) * g.tile[1] * g.tile[2];
 }
@@ -98,12 +98,12 @@ struct ReduceJob {
 };
 
 // True when, in every dimension, a cell is covered only by the tiles of its
-// own bin and its two neighbours: bin >= ns, at least two bins, and the last
-// bin full or at least ns wide. Such geometries use the bin-owned reduction.
+// own bin and its two neighbours: bin >= ns - 1, at least two bins, and the last
+// bin full or at least ns - 1 wide. Such geometries use the bin-owned reduction.
 __host__ __device__ inline bool bins_regular(int dim, const BinGeom& g, int ns) {
   for (int d = 0; d < dim; ++d) {
     const int rem = g.n[d] % g.bin[d];
-    if (g.nbins[d] < 2 || g.bin[d] < ns || (rem != 0 && rem < ns)) return false;
+    if (g.nbins[d] < 2 || g.bin[d] < ns - 1 || (rem != 0 && rem < ns - 1)) return false;
   }
   return true;
 }

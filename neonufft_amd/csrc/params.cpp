@@ -170,7 +170,7 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
   const std::size_t budget = elem_bytes >= 16 ? 144 * 1024 : 100 * 1024;
   auto bytes = [&](const int* b) {
     std::size_t cells = 1;
-    for (int d = 0; d < dim; ++d) cells *= static_cast<std::size_t>(b[d] + ns);
+    for (int d = 0; d < dim; ++d) cells *= static_cast<std::size_t>(b[d] + ns - 1);
     return cells * elem_bytes;
   };
   // shrink the largest bin edge until the LDS tile fits the budget
@@ -181,19 +181,19 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
     if (pref[dmax] <= 1) break;
     pref[dmax] = std::max(1, pref[dmax] / 2);
   }
-  // Prefer bin edges that leave no partial last bin narrower than ns (the tile
+  // Prefer bin edges that leave no partial last bin narrower than ns - 1 (the tile
   // reduction then only needs a bin's direct neighbours): search the nearest
   // edge within max(a quarter of the preferred one, ns) whose tile still fits.
   for (int d = 0; d < dim; ++d) {
     const int nd = static_cast<int>(n[d]);
     const int B = std::min(pref[d], nd);
-    const auto good = [&](int b) { const int r = nd % b; return r == 0 || r >= ns; };
-    if (B < ns || good(B)) continue;
+    const auto good = [&](int b) { const int r = nd % b; return r == 0 || r >= ns - 1; };
+    if (B < ns - 1 || good(B)) continue;
     const int span = std::max(B / 4, ns);
     for (int delta = 1; delta <= span; ++delta) {
       bool found = false;
       for (int cand : {B - delta, B + delta}) {
-        if (cand < ns || cand > nd) continue;
+        if (cand < ns - 1 || cand > nd) continue;
         int trial[3] = {pref[0], pref[1], pref[2]};
         trial[d] = cand;
         if (good(cand) && bytes(trial) <= budget) {
@@ -212,7 +212,7 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
       g.n[d] = nd;
       g.bin[d] = std::max(1, std::min({pref[d], nd, cap}));
       g.nbins[d] = (nd + g.bin[d] - 1) / g.bin[d];
-      g.tile[d] = g.bin[d] + ns;
+      g.tile[d] = g.bin[d] + ns - 1;
     } else {
       g.n[d] = 1;
       g.bin[d] = 1;

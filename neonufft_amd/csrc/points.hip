@@ -24,8 +24,11 @@ inline unsigned grid_for(std::size_t work, int block, unsigned cap = 65535u * 8u
 }
 
 // Fold one coordinate: v = (x - offset) * scale; u = frac((v + pi) / 2 pi);
-// xi = u * n. Returns the containing cell (for the bin), the first kernel
-// cell i0 = ceil(xi - ns/2) and the Horner argument i0 - (xi - ns/2) in [0,1).
+// xi = u * n. Returns the first kernel cell i0 = ceil(xi - ns/2), the Horner
+// argument i0 - (xi - ns/2) in [0,1) and the cell that places the point in a
+// bin: i0 + ns/2 (floor) mod n, so that a bin's points start their kernels on
+// exactly bin cells and its tile needs a halo of ns - 1 (binning by the cell
+// holding xi lets i0 take bin + 1 values). i0 is wrapped along with it.
 __device__ inline void fold_coord(double v, int n, int ns, double& hx, int& i0, int& cell) {
   double u = (v + kPi) / (2.0 * kPi);
   u -= floor(u);
@@ -36,7 +39,11 @@ __device__ inline void fold_coord(double v, int n, int ns, double& hx, int& i0, 
   const double s = ceil(a);
   hx = s - a;
   i0 = static_cast<int>(s);
-  cell = min(static_cast<int>(floor(xi)), n - 1);
+  cell = i0 + ns / 2;
+  if (cell >= n) {
+    cell -= n;
+    i0 -= n;
+  }
 }
 
 template <typename TC, int DIM>

@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(kRowThreads<T>)
     cv.pown = li + h;
     cv.joth = -1;
     cv.poth = 0;
-    if (li < ns - h) {
+    if (li < ns - 1 - h) {
       const int bp = bd == 0 ? nb - 1 : bd - 1;
       cv.joth = entry(bd - 1);
       cv.poth = li + min(g.bin[d], g.n[d] - bp * g.bin[d]) + h;
@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(kRowThreads<T>)
   // Tile rows into the pencil, one x bin per item: the row segment of x bin
   // bx's tiles (every subproblem, own and covering-neighbour y / z tiles)
   // is summed and added to grid cells bx bin0 - ns/2 + j (mod n0),
-  // j < bin width + ns. Consecutive lanes take consecutive j, so tile rows
+  // j < bin width + ns - 1. Consecutive lanes take consecutive j, so tile rows
   // are read coalesced; the first subproblem of every covering tile is
   // loaded before any is waited for. Segments of bins of one parity do not
   // overlap, so the bins are added in two passes (three with an odd bin
@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(kRowThreads<T>)
         const int j = div_rem(i, t0, rt0, &rest);
         const int bxi = div_rem(rest, nbp, rnbp, &r[u]);
         const int bx = phase == 2 ? nb0 - 1 : phase + 2 * bxi;
-        const int ext = min(bin0, n0 - bx * bin0) + ns;
+        const int ext = min(bin0, n0 - bx * bin0) + ns - 1;
         live[u] = i0 + u * NT < items && j < ext;
         int xx = bx * bin0 - h + j;
         x[u] = xx < 0 ? xx + n0 : (xx >= n0 ? xx - n0 : xx);

@@ -7,7 +7,7 @@
 // interpolated value is the same weighted sum over the grid (times the type-3
 // postphase). The design is MI355X-specific:
 //  - one workgroup per subproblem (<= max_points points of one bin), with the
-//    bin's tile plus its ns-cell halo staged in LDS;
+//    bin's tile plus its halo of ns - 1 cells staged in LDS;
 //  - spreading accumulates with LDS atomics, stores the finished tile with
 //    plain coalesced stores, and a tile reduction sums overlapping tiles into
 //    the grid (no global atomics, fixed summation order); interpolation
@@ -53,7 +53,7 @@ struct TileInfo {
       bin /= static_cast<uint32_t>(g.nbins[d]);
       const int o = bc * g.bin[d];
       org[d] = o - NS / 2;
-      ext[d] = min(g.bin[d], g.n[d] - o) + NS;
+      ext[d] = min(g.bin[d], g.n[d] - o) + NS - 1;
     }
     t0 = g.tile[0];
     t1 = DIM >= 2 ? g.tile[1] : 1;
@@ -577,10 +577,10 @@ __device__ inline void reduce_row(const ReduceJob<T, DIM>& job, int c1, int c2, 
 }
 
 // ---------------------------------------------------------------------------
-// Bin-owned tile reduction for regular geometries (per dimension: bin >= ns,
-// at least two bins, last bin full or >= ns wide). Then a cell of bin b is
+// Bin-owned tile reduction for regular geometries (per dimension: bin >=
+// ns - 1, at least two bins, last bin full or >= ns - 1 wide). Then a cell of bin b is
 // covered only by the tiles of b and of its two neighbours: by b at position
-// i + ns/2 (i = offset inside the bin), by b - 1 when i < ns - ns/2 (at
+// i + ns/2 (i = offset inside the bin), by b - 1 when i < ns - 1 - ns/2 (at
 // i + w(b - 1) + ns/2) and by b + 1 when i >= w(b) - ns/2 (at
 // i - w(b) + ns/2), w = bin width, neighbours periodic. One workgroup takes
 // one bin: the subproblem ranges of the 3^DIM neighbour bins go to LDS once,
@@ -642,7 +642,7 @@ __device__ inline void reduce_bin(const ReduceJob<T, DIM>& job, int ns, uint32_t
 #pragma unroll
       for (int d = 0; d < DIM; ++d) {
         pown[d] = li[d] + h;
-        if (li[d] < ns - h) {
+        if (li[d] < ns - 1 - h) {
           ooth[d] = -1;
           poth[d] = li[d] + wprev[d] + h;
         } else if (li[d] >= w[d] - h) {
