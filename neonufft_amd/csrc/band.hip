@@ -391,7 +391,7 @@ __global__ void __launch_bounds__(kBandThreads<T>)
       const int x0 = static_cast<int>(rec[k].cell & CellPack<2>::mask) - NS / 2;
       const int l0 = valid ? static_cast<int>(rec[k].cell >> CellPack<2>::bits) + lr0[k] : rk;
       T kx[NS];
-      es_weights<T, NS>(rec[k].x[0], es, kx);
+      es_weights<NS>(rec[k].x[0], es, kx);
       // cells x0 .. x0 + NS - 1 of the row, unwrapped: a run that crosses
       // either end of the row lands in the row's halo and is folded below,
       // so the NS atomics of a row share one address register

@@ -59,8 +59,36 @@ __device__ inline double es_piece(double x, int j, const EsParams& es) {
   return a > 0.0 ? exp(es.beta * (sqrt(a) - 1.0)) : 0.0;
 }
 
-template <typename T, int NS>
-__device__ inline void es_weights(T x, const EsParams& es, T (&k)[NS]) {
+// All NS weights of one axis. The kernel is even, so piece NS - 1 - j at y is
+// piece j at -y: each pair shares the even part E(y^2) and the odd part
+// y O(y^2) of one polynomial, and the middle piece of an odd width is its even
+// part (8 instead of 14 FMAs per pair at NS = 6).
+template <int NS>
+__device__ inline void es_weights(float x, const EsParams& es, float (&k)[NS]) {
+  constexpr int DEG = horner_degree(NS);
+  constexpr int ETOP = DEG & ~1, OTOP = (DEG - 1) | 1;
+  const float y = fmaf(2.0f, x, -1.0f);
+  const float y2 = y * y;
+#pragma unroll
+  for (int j = 0; j < (NS + 1) / 2; ++j) {
+    const float* c = es.coef + j * (DEG + 1);
+    float e = c[ETOP];
+#pragma unroll
+    for (int d = ETOP - 2; d >= 0; d -= 2) e = fmaf(e, y2, c[d]);
+    if (2 * j + 1 == NS) {
+      k[j] = e;
+    } else {
+      float o = c[OTOP];
+#pragma unroll
+      for (int d = OTOP - 2; d >= 1; d -= 2) o = fmaf(o, y2, c[d]);
+      k[j] = fmaf(y, o, e);
+      k[NS - 1 - j] = fmaf(-y, o, e);
+    }
+  }
+}
+
+template <int NS>
+__device__ inline void es_weights(double x, const EsParams& es, double (&k)[NS]) {
 #pragma unroll
   for (int j = 0; j < NS; ++j) k[j] = es_piece<NS>(x, j, es);
 }

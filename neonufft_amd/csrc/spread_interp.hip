@@ -60,6 +60,11 @@ struct TileInfo {
   }
 };
 
+// z weights formed in pairs ahead of the z loop where that loop is unrolled
+// and the weights are polynomials; otherwise one per iteration.
+template <typename T, int NS>
+constexpr bool kPairZ = sizeof(T) == 4 && NS <= 8;
+
 // Sum over the workgroup; contains a __syncthreads().
 template <typename T>
 __device__ inline T block_sum(T v, T* scratch) {
@@ -126,7 +131,7 @@ __device__ __forceinline__ void spread_subproblem(const SpreadJob<T, DIM>& job,
     if (p >= end) continue;
     const Cplx<T> c{cv[k].x * scale, cv[k].y * scale};
     T kx[NS];
-    es_weights<T, NS>(rec[k].x[0], es, kx);
+    es_weights<NS>(rec[k].x[0], es, kx);
     const int r0 = unpack_cell<DIM>(rec[k].cell, 0);
     if constexpr (DIM == 1) {
 #pragma unroll
@@ -140,16 +145,18 @@ __device__ __forceinline__ void spread_subproblem(const SpreadJob<T, DIM>& job,
       }
     } else {
       T ky[NS];
-      es_weights<T, NS>(rec[k].x[1], es, ky);
+      es_weights<NS>(rec[k].x[1], es, ky);
       const int r1 = unpack_cell<DIM>(rec[k].cell, 1);
       int r2 = 0;
       if constexpr (DIM == 3) r2 = unpack_cell<DIM>(rec[k].cell, 2);
       constexpr int NZ = DIM == 3 ? NS : 1;
       constexpr int kUnrollZ = NS <= 8 ? NZ : 1;
+      T kz[NS];
+      if constexpr (DIM == 3 && kPairZ<T, NS>) es_weights<NS>(rec[k].x[2], es, kz);
 #pragma unroll kUnrollZ
       for (int cz = 0; cz < NZ; ++cz) {
         T wz = T(1);
-        if constexpr (DIM == 3) wz = es_piece<NS>(rec[k].x[2], cz, es);
+        if constexpr (DIM == 3) wz = kPairZ<T, NS> ? kz[cz] : es_piece<NS>(rec[k].x[2], cz, es);
         const T czr = wz * c.x, czi = wz * c.y;
 #pragma unroll
         for (int b = 0; b < NS; ++b) {
@@ -320,7 +327,7 @@ __device__ __forceinline__ void interp_subproblem(const InterpJob<T, DIM>& job,
   for (uint32_t p = sp.begin + threadIdx.x; p < end; p += kInterpThreads<T>) {
     const PointRec<T, DIM> rec = pts[p];
     T kx[NS];
-    es_weights<T, NS>(rec.x[0], es, kx);
+    es_weights<NS>(rec.x[0], es, kx);
     const int r0 = unpack_cell<DIM>(rec.cell, 0);
     T sr = T(0), si = T(0);
     if constexpr (DIM == 1) {
@@ -332,7 +339,7 @@ __device__ __forceinline__ void interp_subproblem(const InterpJob<T, DIM>& job,
       }
     } else {
       T ky[NS];
-      es_weights<T, NS>(rec.x[1], es, ky);
+      es_weights<NS>(rec.x[1], es, ky);
       const int r1 = unpack_cell<DIM>(rec.cell, 1);
       int r2 = 0;
       if constexpr (DIM == 3) r2 = unpack_cell<DIM>(rec.cell, 2);
@@ -341,6 +348,8 @@ __device__ __forceinline__ void interp_subproblem(const InterpJob<T, DIM>& job,
       // ahead of the FMAs and spill them; unroll z in fp32 only, y by 2.
       constexpr int kUnrollZ = (sizeof(T) == 4 && NS <= 8) ? NZ : 1;
       constexpr int kUnrollY = sizeof(T) == 4 ? NS : 2;
+      T kz[NS];
+      if constexpr (DIM == 3 && kPairZ<T, NS>) es_weights<NS>(rec.x[2], es, kz);
 #pragma unroll kUnrollZ
       for (int cz = 0; cz < NZ; ++cz) {
         T pr = T(0), pi = T(0);
@@ -358,7 +367,7 @@ __device__ __forceinline__ void interp_subproblem(const InterpJob<T, DIM>& job,
           pi += ky[b] * ri;
         }
         T wz = T(1);
-        if constexpr (DIM == 3) wz = es_piece<NS>(rec.x[2], cz, es);
+        if constexpr (DIM == 3) wz = kPairZ<T, NS> ? kz[cz] : es_piece<NS>(rec.x[2], cz, es);
         sr += wz * pr;
         si += wz * pi;
       }
