@@ -43,5 +43,10 @@ def test_edges(prec, dim, modes, tol):
     # the same algorithm in FP64; fp32 adds its rounding (bound of the fp32
     # share of every parity test: 3e-6 + 0.04 tol)
     bound = 3e-6 + 0.04 * tol if prec == "f32" else 1e-10
+    # an even kernel ends on whole cells, where it jumps from exp(-beta) to 0:
+    # a point there keeps or loses that weight, per axis, with the last bit of
+    # its folded coordinate (beta = 2.3 ns)
+    if prec == "f64" and tol == 1e-5:
+        bound = dim * np.exp(-2.3 * 6)
     assert O.rel_l2(out.cpu().numpy(), O.nufft1(x64, c.astype(np.complex128), modes, -1, tol)) < bound
     assert O.rel_l2(back.cpu().numpy(), O.nufft2(x64, f.astype(np.complex128), modes, -1, tol)) < bound
