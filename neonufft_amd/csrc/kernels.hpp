@@ -160,6 +160,33 @@ void launch_interp_batch(int ns, const InterpJob<T, DIM>* jobs, const Subprob* s
                          std::size_t nsub, std::size_t lds_bytes, const EsParams& es,
                          hipStream_t stream);
 
+// ---- planes.hip: 3D fp64 spreading / interpolation on the matrix cores ------
+// Tiles of at most 16 x 16 cells in x and y take it, kernels up to 12 cells
+// wide (a wider one leaves bins of four cells and fewer in a 16-cell tile).
+constexpr int kPlaneCells = 16;
+constexpr int kPlaneMaxWidth = 12;
+constexpr int kMaxTilePlanes = 64;  // planes of one tile
+
+// True when the points of geometry g are ordered by first kernel plane and
+// spread / interpolated by the plane kernels.
+template <typename T, int DIM>
+bool plane_tiles(const BinGeom& g, int ns) {
+  return std::is_same_v<T, double> && DIM == 3 && ns <= kPlaneMaxWidth &&
+         g.tile[0] <= kPlaneCells && g.tile[1] <= kPlaneCells &&
+         g.tile[2] <= kMaxTilePlanes;
+}
+
+void launch_plane_order(const Subprob* subs, std::size_t nsub, PointRec<double, 3>* pts,
+                        uint32_t* perm, hipStream_t stream);
+void launch_plane_spread(int ns, const SpreadJob<double, 3>& job, const Subprob* subs,
+                         std::size_t nsub, const EsParams& es, hipStream_t stream);
+void launch_plane_interp(int ns, const InterpJob<double, 3>& job, const Subprob* subs,
+                         std::size_t nsub, const EsParams& es, hipStream_t stream);
+void launch_plane_spread_batch(int ns, const SpreadJob<double, 3>* jobs, const Subprob* subs,
+                               std::size_t nsub, const EsParams& es, hipStream_t stream);
+void launch_plane_interp_batch(int ns, const InterpJob<double, 3>* jobs, const Subprob* subs,
+                               std::size_t nsub, const EsParams& es, hipStream_t stream);
+
 // Dynamic LDS bytes of one spreading / interpolation block for a bin geometry.
 template <typename T>
 std::size_t tile_bytes(const BinGeom& g);

@@ -140,7 +140,7 @@ int band_rows(IntType n0, IntType pitch, IntType n1, int ns, std::size_t acc_byt
 }
 
 BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
-                    const int* bin_override) {
+                    const int* bin_override, bool planes) {
   BinGeom g{};
   int pref[3] = {1, 1, 1};
   // Defaults measured on MI355X for uniform points at ~0.6 points per cell
@@ -157,9 +157,21 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
     pref[1] = 8;
     pref[2] = 8;
   }
+  bool overridden = false;
   if (bin_override) {
-    for (int d = 0; d < dim; ++d)
-      if (bin_override[d] > 0) pref[d] = bin_override[d];
+    for (int d = 0; d < dim; ++d) {
+      if (bin_override[d] > 0) {
+        pref[d] = bin_override[d];
+        overridden = true;
+      }
+    }
+  }
+  int most[3] = {1 << 30, 1 << 30, 1 << 30};
+  if (dim == 3 && elem_bytes >= 16 && ns <= kPlaneMaxWidth && planes && !overridden) {
+    // fp64 plane kernels: tiles of 16 x 16 cells
+    most[0] = most[1] = pref[0] = pref[1] = kPlaneCells + 1 - ns;
+    most[2] = kMaxTilePlanes + 1 - ns;
+    pref[2] = 32 + 1 - ns;
   }
   // LDS tile bytes per workgroup (160 KB per CU on gfx950). Measured on MI355X
   // with 128^3 modes: fp64 tiles need most of it, since at ns >= 9 a 60 KB
@@ -193,7 +205,7 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
     for (int delta = 1; delta <= span; ++delta) {
       bool found = false;
       for (int cand : {B - delta, B + delta}) {
-        if (cand < ns - 1 || cand > nd) continue;
+        if (cand < ns - 1 || cand > nd || cand > most[d]) continue;
         int trial[3] = {pref[0], pref[1], pref[2]};
         trial[d] = cand;
         if (good(cand) && bytes(trial) <= budget) {

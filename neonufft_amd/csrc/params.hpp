@@ -40,8 +40,9 @@ double fit_horner(int ns, double beta, int deg, double* coef /* ns*(deg+1) */);
 
 // Bin geometry for a grid of size n (DIM entries), element size and ns.
 // bin_override: if non-null and positive entries, used instead of the default.
+// planes: 3D fp64 defaults suit the plane kernels (planes.hip).
 BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
-                    const int* bin_override = nullptr);
+                    const int* bin_override = nullptr, bool planes = true);
 
 // Rows per band of the row-band spreading of an n0 x n1 grid with LDS rows of
 // `pitch` cells: as many as two accumulator planes (acc_bytes per cell) of

@@ -89,7 +89,12 @@ public:
     launch_subprob_build(t.count, t.start, t.sub_start, nbins, max_points, subs_.data(), stream);
     launch_bin_scatter<TC, T, DIM>(loc, m, fp, g, ns, t.start, t.rank, recs_.data(), perm_.data(),
                                    stream);
-    launch_bank_order<T, DIM>(subs_.data(), nsub_, recs_.data(), perm_.data(), g, stream);
+    bool ordered = false;
+    if constexpr (std::is_same_v<T, double> && DIM == 3) {
+      ordered = plane_tiles<T, DIM>(g, ns);
+      if (ordered) launch_plane_order(subs_.data(), nsub_, recs_.data(), perm_.data(), stream);
+    }
+    if (!ordered) launch_bank_order<T, DIM>(subs_.data(), nsub_, recs_.data(), perm_.data(), g, stream);
     if (ws) {
       check_hip(hipMemcpyAsync(sub_start_.data(), t.sub_start, (nbins + 1) * sizeof(uint32_t),
                                hipMemcpyDeviceToDevice, stream),

@@ -824,6 +824,12 @@ void launch_spread(int ns, const PointRec<T, DIM>* pts, const uint32_t* perm, co
                    const BinGeom& g, const EsParams& es, hipStream_t stream) {
   if (nsub == 0) return;
   const SpreadJob<T, DIM> job{pts, perm, in, pre_sorted, tiles, 0u, 0u, g};
+  if constexpr (std::is_same_v<T, double> && DIM == 3) {
+    if (plane_tiles<T, DIM>(g, ns)) {
+      launch_plane_spread(ns, job, subs, nsub, es, stream);
+      return;
+    }
+  }
   NNF_NS_CASES(spread_ns, job, subs, nsub, es, stream)
 }
 
@@ -833,6 +839,12 @@ void launch_interp(int ns, const PointRec<T, DIM>* pts, const uint32_t* perm, co
                    const BinGeom& g, const EsParams& es, hipStream_t stream) {
   if (nsub == 0) return;
   const InterpJob<T, DIM> job{pts, perm, grid, post_sorted, out, g};
+  if constexpr (std::is_same_v<T, double> && DIM == 3) {
+    if (plane_tiles<T, DIM>(g, ns)) {
+      launch_plane_interp(ns, job, subs, nsub, es, stream);
+      return;
+    }
+  }
   NNF_NS_CASES(interp_ns, job, subs, nsub, es, stream)
 }
 
