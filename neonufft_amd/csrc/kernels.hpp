@@ -304,7 +304,14 @@ struct RowFftJob {
   Cplx<T>* grid;              // type 2: fine grid written (x fastest)
   const Cplx<T>* tw;          // twiddles as for the row bands (tw[N/2 + q])
   int N0, log2n0, rows, log2rows, pitch;
+  // One word per pencil, z * ceil(n1 / rows) + y / rows: non-zero where the
+  // tile of a bin with points meets it; null = every pencil counts.
+  const uint32_t* used;
 };
+// used[pencil] = 1 for the pencils above; `used` is zero beforehand.
+template <int DIM>
+void launch_mark_pencils(const uint32_t* sub_start, const BinGeom& g, int ns, int rows,
+                         uint32_t* used, hipStream_t stream);
 // Entries of a reduction pencil's subproblem-range table: every x bin x the y
 // bins its rows meet plus one on each side x three z bins (3D).
 inline int row_fft_rng_entries(const BinGeom& g, int rows, int dim) {

@@ -187,6 +187,13 @@ public:
     // to the zero padding (type 2); NNF_SPREAD_TILES keeps the separate
     // reduction, rocFFT x pass and transposes
     if (tune_.spread_mode != kSpreadTiles) row_rows_ = row_fft_rows(DIM, geom_, sizeof(T));
+    if constexpr (DIM >= 2) {
+      if (row_rows_ > 0) {
+        pencils_ = static_cast<std::size_t>((n_[1] + row_rows_ - 1) / row_rows_) *
+                   static_cast<std::size_t>(n_[2]);
+        used_.reset(pencils_, alloc_);
+      }
+    }
     // 3D with the row kernels: the y and z passes in LDS too, when both
     // extents are powers of two >= 32
     IntType tw_len = n_[0];
@@ -238,6 +245,13 @@ public:
     points_valid_ = false;
     pts_.build(l, m, fp, geom_, ks_.ns, tune_.max_points, stream_, alloc_, ws);
     bands_on_ = false;
+    if constexpr (DIM >= 2) {
+      if (row_rows_ > 0) {
+        launch_fill_u32(used_.data(), pencils_, 0u, stream_);
+        launch_mark_pencils<DIM>(pts_.sub_starts(), geom_, ks_.ns, row_rows_, used_.data(),
+                                 stream_);
+      }
+    }
     if constexpr (DIM == 2) {
       if (band_rows_ > 0) {
         if (ws) ws->used = 0;  // the point set's temporaries are no longer needed
@@ -318,6 +332,8 @@ public:
   }
   void reduce_tiles(bool accumulate) {
     require_points();
+    if (accumulate) complete_grid();
+    grid_partial_ = false;
     if constexpr (DIM == 2) {
       if (bands_on_) {
         const int nb = static_cast<int>((n_[1] + band_rows_ - 1) / band_rows_);
@@ -335,6 +351,11 @@ public:
 
   // Stage 3 of type 2: interpolate the current fine grid.
   void interp(Cplx<T>* out) {
+    complete_grid();
+    interp_points(out);
+  }
+
+  void interp_points(Cplx<T>* out) {
     require_points();
     if (pts_.size() && !out) throw neonufft::InputError("Neonufft:: null output");
     launch_interp<T, DIM>(ks_.ns, pts_.recs(), pts_.perm(), pts_.subs(), pts_.nsub(), grid_.data(),
@@ -344,6 +365,7 @@ public:
   void transform_type_1(const Cplx<T>* in, Cplx<T>* out, const IntType* out_strides) {
     require_points();
     if (!out || !out_strides) throw neonufft::InputError("Neonufft:: null output");
+    grid_partial_ = false;  // the grid is work memory again, h is overwritten
     T* fs[3] = {fs_[0].data(), fs_[1].data(), fs_[2].data()};
     if constexpr (DIM == 2) {
       if (bands_on_ && band_.fft) {
@@ -365,7 +387,7 @@ public:
       if (row_rows_ > 0 && !bands_on_ && bins_regular(DIM, geom_, ks_.ns)) {
         // tiles -> retained x modes in one pass, then the remaining passes
         spread_tiles(in);
-        launch_reduce_rows_fft<T, DIM>(row_job(), ks_.ns, stream_);
+        launch_reduce_rows_fft<T, DIM>(row_job(used_.data()), ks_.ns, stream_);
         if (axis_rows_y_ > 0) {
           launch_axis_fft_type1<T>(axis_job(out, nullptr, out_strides), stream_);
         } else {
@@ -400,12 +422,14 @@ public:
         } else {
           pfft_.backward_to_h(in, nullptr, in_strides, fs, order_fft(), stream_);
         }
-        launch_expand_rows_ifft<T>(row_job(), stream_);
+        // only the rows that points read, unless the caller has asked for the grid
+        launch_expand_rows_ifft<T>(row_job(grid_shown_ ? nullptr : used_.data()), stream_);
+        grid_partial_ = !grid_shown_;
       } else {
         pfft_.backward(in, nullptr, in_strides, fs, order_fft(), grid_.data(), stream_);
       }
     }
-    interp(out);
+    interp_points(out);
   }
 
   void info(nnf_plan_info* info) const {
@@ -429,7 +453,12 @@ public:
     info->band_rows = bands_on_ ? band_rows_ : 0;
   }
 
-  Cplx<T>* fine_grid() const { return grid_.data(); }
+  // From here on type 2 forms every row of the grid: the caller may read it.
+  Cplx<T>* fine_grid() {
+    complete_grid();
+    grid_shown_ = true;
+    return grid_.data();
+  }
   const T* fseries(int d) const { return d >= 0 && d < DIM ? fs_[d].data() : nullptr; }
 
 private:
@@ -477,8 +506,17 @@ private:
     return j;
   }
 
-  RowFftJob<T> row_job() const {
+  // The rows that the last type 2 left out, from the h it left behind.
+  void complete_grid() {
+    if constexpr (DIM >= 2) {
+      if (grid_partial_) launch_expand_rows_ifft<T>(row_job(nullptr), stream_);
+    }
+    grid_partial_ = false;
+  }
+
+  RowFftJob<T> row_job(const uint32_t* used) const {
     RowFftJob<T> j{};
+    j.used = used;
     j.tiles = tiles_.data();
     j.sub_start = pts_.sub_starts();
     j.g = geom_;
@@ -536,6 +574,10 @@ private:
   int axis_rows_y_ = 0;           // 3D: lines per workgroup of the LDS y pass (0 = rocFFT)
   int axis_rows_z_ = 0;           // 3D: lines per workgroup of the LDS z pass
   bool bands_on_ = false;         // row bands used for the current points
+  std::size_t pencils_ = 0;       // pencils of the row kernels
+  DeviceBuffer<uint32_t> used_;   // pencils that the tiles of the points meet
+  bool grid_partial_ = false;     // the grid lacks the rows no point reads
+  bool grid_shown_ = false;       // fine_grid() has handed out the grid
   bool points_valid_ = false;     // the last set_points succeeded
   std::vector<uint32_t> row_host_;  // row offsets of the view (balance check)
   BandLayout band_;

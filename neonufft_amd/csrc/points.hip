@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(kScanThreads)
     s += v[k];
   }
   uint32_t tot;
-  uint32_t run = tile_off[blockIdx.x] + block_exclusive_scan(s, &tot);
+  uint32_t run = (tile_off ? tile_off[blockIdx.x] : 0u) + block_exclusive_scan(s, &tot);
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
     if (base + k < n) out[base + k] = run;
@@ -372,6 +372,12 @@ void launch_exclusive_scan(const uint32_t* in, uint32_t* out, std::size_t n, uin
                            hipStream_t stream) {
   if (n == 0) return;
   const std::size_t tiles = (n + kScanTile - 1) / kScanTile;
+  if (tiles == 1) {  // one launch instead of three (~3 us each)
+    hipLaunchKernelGGL(scan_tiles_kernel, dim3(1), dim3(kScanThreads), 0, stream, in, n,
+                       static_cast<const uint32_t*>(nullptr), out);
+    check_launch("scan_tiles_kernel");
+    return;
+  }
   hipLaunchKernelGGL(scan_tile_sums, dim3(static_cast<unsigned>(tiles)), dim3(kScanThreads), 0,
                      stream, in, n, scratch);
   check_launch("scan_tile_sums");

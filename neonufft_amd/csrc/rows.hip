@@ -46,6 +46,33 @@ __device__ inline void batched_copy(int total, Load load, Store store) {
   }
 }
 
+// Thread per bin: the pencils its tile meets, if it has points.
+template <int DIM>
+__global__ void __launch_bounds__(256)
+    mark_pencils_kernel(const uint32_t* __restrict__ sub_start, BinGeom g, int ns, int rows,
+                        uint32_t* __restrict__ used) {
+  const uint32_t nbins = static_cast<uint32_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2];
+  const uint32_t b = threadIdx.x + blockIdx.x * 256u;
+  if (b >= nbins || sub_start[b + 1] == sub_start[b]) return;
+  const uint32_t yz = b / static_cast<uint32_t>(g.nbins[0]);
+  const int oy = static_cast<int>(yz % static_cast<uint32_t>(g.nbins[1])) * g.bin[1];
+  const int oz = static_cast<int>(yz / static_cast<uint32_t>(g.nbins[1])) * g.bin[2];
+  const int ey = min(min(g.bin[1], g.n[1] - oy) + ns - 1, g.n[1]);
+  const int ez = DIM >= 3 ? min(min(g.bin[2], g.n[2] - oz) + ns - 1, g.n[2]) : 1;
+  const int groups = (g.n[1] + rows - 1) / rows;
+  for (int z = 0; z < ez; ++z) {
+    const int gz = DIM >= 3 ? wrap_once(oz - ns / 2 + z, g.n[2]) : 0;
+    for (int y = 0; y < ey; ++y) used[gz * groups + wrap_once(oy - ns / 2 + y, g.n[1]) / rows] = 1u;
+  }
+}
+
+// True when the pencil of this workgroup meets no tile (uniform).
+template <typename T>
+__device__ inline bool pencil_unused(const RowFftJob<T>& job, int z, int y0) {
+  const int groups = (job.g.n[1] + job.rows - 1) / job.rows;
+  return job.used && job.used[z * groups + (y0 >> job.log2rows)] == 0u;
+}
+
 // Pencil of workgroup blockIdx.x: rows [y0, y0 + rk) of plane z. Pencils
 // next to each other in y and z (which read the same halo tiles) go to one
 // XCD and so meet in its L2.
@@ -71,6 +98,15 @@ __global__ void __launch_bounds__(kRowThreads<T>)
   const BinGeom& g = job.g;
   const int n0 = g.n[0], n1 = g.n[1];
   const Pencil pc = pencil_of(job.rows, n1);
+  if (pencil_unused(job, pc.z, pc.y0)) {
+    // no tile: its rows and their modes are zero
+    Cplx<T>* __restrict__ hz = job.h + static_cast<std::size_t>(pc.z) * job.N0 * n1 + pc.y0;
+    for (int i = threadIdx.x; i < (job.N0 << job.log2rows); i += NT) {
+      const int r = i & (job.rows - 1);
+      if (r < pc.rk) hz[static_cast<std::size_t>(i >> job.log2rows) * n1 + r] = Cplx<T>{T(0), T(0)};
+    }
+    return;
+  }
   T* fre = reinterpret_cast<T*>(smem_raw);
   T* fim = fre + job.rows * job.pitch;
   // subproblem ranges of the bins the pencil's cells can meet: every x bin,
@@ -270,6 +306,7 @@ __global__ void __launch_bounds__(kRowThreads<T>) expand_rows_ifft_kernel(RowFft
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int n0 = job.g.n[0], n1 = job.g.n[1];
   const Pencil pc = pencil_of(job.rows, n1);
+  if (pencil_unused(job, pc.z, pc.y0)) return;  // no point reads its rows
   T* fre = reinterpret_cast<T*>(smem_raw);
   T* fim = fre + job.rows * job.pitch;
   for (int i = threadIdx.x; i < 2 * job.rows * job.pitch; i += NT) fre[i] = T(0);
@@ -624,6 +661,19 @@ void launch_expand_rows_ifft(const RowFftJob<T>& job, hipStream_t stream) {
                      dim3(kRowThreads<T>), lds, stream, job);
   check_launch("expand_rows_ifft_kernel");
 }
+
+template <int DIM>
+void launch_mark_pencils(const uint32_t* sub_start, const BinGeom& g, int ns, int rows,
+                         uint32_t* used, hipStream_t stream) {
+  const std::size_t nbins = static_cast<std::size_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2];
+  hipLaunchKernelGGL((mark_pencils_kernel<DIM>), dim3(static_cast<unsigned>((nbins + 255) / 256)),
+                     dim3(256), 0, stream, sub_start, g, ns, rows, used);
+  check_launch("mark_pencils_kernel");
+}
+template void launch_mark_pencils<2>(const uint32_t*, const BinGeom&, int, int, uint32_t*,
+                                     hipStream_t);
+template void launch_mark_pencils<3>(const uint32_t*, const BinGeom&, int, int, uint32_t*,
+                                     hipStream_t);
 
 template void launch_reduce_rows_fft<float, 2>(const RowFftJob<float>&, int, hipStream_t);
 template void launch_reduce_rows_fft<float, 3>(const RowFftJob<float>&, int, hipStream_t);
