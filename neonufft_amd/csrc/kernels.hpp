@@ -22,6 +22,9 @@ struct QuadRule {
   int nq;
 };
 
+// Longest axis of the summed transforms of small plans (pruned.hip).
+constexpr int kDftMaxLen = 128;
+
 // Upper bound on the points of one subproblem (one workgroup's worth).
 constexpr uint32_t kMaxSubproblemPoints = 2048;
 

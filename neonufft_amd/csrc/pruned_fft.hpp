@@ -12,7 +12,10 @@
 // the LDS axis kernels of rows.hip and use only the h() and k() arrays.
 #pragma once
 
+#include <algorithm>
+#include <cmath>
 #include <memory>
+#include <vector>
 
 #include "fft.hpp"
 #include "kernels.hpp"
@@ -41,6 +44,26 @@ void launch_modes_in(const Cplx<T>* single, const Cplx<T>* const* ins, int count
                      long long stm, long long stl, const T* fs0, const T* fsm, const T* fsl,
                      int order_fft, hipStream_t stream);
 
+// Summed transforms of small fp32 axes, each with the step before or after it:
+// FFT + compact transpose (keep) or expanding transpose + FFT; FFT + modes_out;
+// modes_in + FFT. At most 65535 slabs, n <= kDftMaxLen.
+void launch_dft_move(bool keep, const double2* tw, const Cplx<float>* src, Cplx<float>* dst, int R,
+                     int n, int N, long long src_rs, long long dst_rs, std::size_t slabs,
+                     int lo_count, long long src_hi, long long src_lo, long long dst_hi,
+                     long long dst_lo, hipStream_t stream);
+template <int DIM>
+void launch_dft_modes_out(const double2* tw, const Cplx<float>* src, long long member_stride,
+                          Cplx<float>* single, Cplx<float>* const* outs, int count, int N0, int Nm,
+                          int nl, int Nl, long long st0, long long stm, long long stl,
+                          const float* fs0, const float* fsm, const float* fsl, int order_fft,
+                          hipStream_t stream);
+template <int DIM>
+void launch_dft_modes_in(const double2* tw, const Cplx<float>* single,
+                         const Cplx<float>* const* ins, int count, Cplx<float>* dst,
+                         long long member_stride, int N0, int Nm, int nl, int Nl, long long st0,
+                         long long stm, long long stl, const float* fs0, const float* fsm,
+                         const float* fsl, int order_fft, hipStream_t stream);
+
 // DIM 2 or 3 (1D plans transform their single axis directly).
 template <typename T, int DIM>
 class PrunedFft {
@@ -63,16 +86,21 @@ public:
     if (DIM == 2 && n_[1] >= 32 && (n_[1] & (n_[1] - 1)) == 0) {
       y_rows_ = axis_fft_rows(static_cast<IntType>(n_[1]), sizeof(T), kBandBudget);
     }
+    h_.reset(static_cast<std::size_t>(count * n_[2] * N_[0] * n_[1]), alloc);
+    if (DIM == 3) k_.reset(static_cast<std::size_t>(count * N_[1] * N_[0] * n_[2]), alloc);
+    small_ = small_axes();
+    if (small_) {
+      upload_dft_twiddles(sign, stream, alloc);
+      return;
+    }
     const bool dbl = std::is_same_v<T, double>;
     IntType len = n_[0];
     px_ = FftPlan(dbl, 1, &len, sign, static_cast<IntType>(count * n_[1] * n_[2]), stream, alloc);
     len = n_[1];
     py_ = FftPlan(dbl, 1, &len, sign, static_cast<IntType>(count * n_[2] * N_[0]), stream, alloc);
-    h_.reset(static_cast<std::size_t>(count * n_[2] * N_[0] * n_[1]), alloc);
     if (DIM == 3) {
       len = n_[2];
       pz_ = FftPlan(dbl, 1, &len, sign, static_cast<IntType>(count * N_[1] * N_[0]), stream, alloc);
-      k_.reset(static_cast<std::size_t>(count * N_[1] * N_[0] * n_[2]), alloc);
     }
   }
 
@@ -90,7 +118,6 @@ public:
   // deconvolution into the outputs.
   void forward_from_h(T* const* fs, int order_fft, Cplx<T>* single, Cplx<T>* const* outs,
                       const IntType* st, hipStream_t s) {
-    py_.execute(h_.data());
     finish_forward(fs, order_fft, single, outs, st, s);
   }
 
@@ -134,6 +161,26 @@ public:
   void backward_to_h(const Cplx<T>* single, const Cplx<T>* const* ins, const IntType* st,
                      T* const* fs, int order_fft, hipStream_t s) {
     const long long n1 = n_[1], n2 = n_[2], N0 = N_[0], N1 = N_[1], N2 = N_[2];
+    if constexpr (std::is_same_v<T, float>) {
+      if (small_) {
+        if constexpr (DIM == 2) {
+          launch_dft_modes_in<2>(dft(1), single, ins, count_, h_.data(), N0 * n1,
+                                 static_cast<int>(N0), 1, static_cast<int>(n1),
+                                 static_cast<int>(N1), st[0], 0, st[1], fs[0], fs[1], fs[1],
+                                 order_fft, s);
+        } else {
+          launch_dft_modes_in<3>(dft(2), single, ins, count_, k_.data(), N1 * N0 * n2,
+                                 static_cast<int>(N0), static_cast<int>(N1), static_cast<int>(n2),
+                                 static_cast<int>(N2), st[0], st[1], st[2], fs[0], fs[1], fs[2],
+                                 order_fft, s);
+          launch_dft_move(false, dft(1), k_.data(), h_.data(), static_cast<int>(n2),
+                          static_cast<int>(n1), static_cast<int>(N1), N0 * n2, N0 * n1,
+                          static_cast<std::size_t>(count_ * N0), static_cast<int>(N0),
+                          N1 * N0 * n2, n2, n2 * N0 * n1, n1, s);
+        }
+        return;
+      }
+    }
     if constexpr (DIM == 2) {
       launch_modes_in<T, 2>(single, ins, count_, h_.data(), N0 * n1, static_cast<int>(N0), 1,
                             static_cast<int>(n1), static_cast<int>(N1), st[0], 0, st[1], fs[0],
@@ -152,6 +199,7 @@ public:
   }
 
   void set_stream(hipStream_t s) {
+    if (small_) return;
     px_.set_stream(s);
     py_.set_stream(s);
     if (DIM == 3) pz_.set_stream(s);
@@ -163,12 +211,20 @@ public:
                Cplx<T>* const* outs, const IntType* st, hipStream_t s) {
     const long long n0 = n_[0], n1 = n_[1], n2 = n_[2], N0 = N_[0];
     const long long gstride = n0 * n1 * n2;
+    if constexpr (std::is_same_v<T, float>) {
+      if (small_) {
+        launch_dft_move(true, dft(0), grids, h_.data(), static_cast<int>(n1), static_cast<int>(n0),
+                        static_cast<int>(N0), n0, n1, static_cast<std::size_t>(count_ * n2),
+                        static_cast<int>(n2), gstride, n1 * n0, n2 * N0 * n1, N0 * n1, s);
+        finish_forward(fs, order_fft, single, outs, st, s);
+        return;
+      }
+    }
     px_.execute(grids);
     launch_compact_transpose<T>(grids, h_.data(), static_cast<int>(n1), static_cast<int>(n0),
                                 static_cast<int>(N0), n0, n1,
                                 static_cast<std::size_t>(count_ * n2), static_cast<int>(n2),
                                 gstride, n1 * n0, n2 * N0 * n1, N0 * n1, s);
-    py_.execute(h_.data());
     finish_forward(fs, order_fft, single, outs, st, s);
   }
 
@@ -181,12 +237,57 @@ public:
   }
 
 private:
-  // After the y-FFT of h: 2D deconvolves from h; 3D transposes to K, runs the
-  // z-FFT and deconvolves.
+  // fp32 transforms small enough for summed axes: no axis above kDftMaxLen and
+  // at most kDftMaxSums products in all passes (2 n0 n1 n2 N0 and so on).
+  // Type 2 of 3000 points, us, library passes -> sums: 12 x 10 x 11 modes 28 -> 19,
+  // 28 x 27 x 26 29 -> 24, 31 x 30 x 29 47 -> 26, 33 x 31 x 30 38 -> 27, and
+  // nothing gained at 36 x 35 x 34 (2.1e7 products). Type 1 in 2D: 50 x 40 27 ->
+  // 26, 70 x 60 28 -> 29, 120 x 100 29 -> 35: axes end at 128 cells.
+  static constexpr double kDftMaxSums = 16777216.0;
+  bool small_axes() const {
+    if (!std::is_same_v<T, float>) return false;
+    double sums = 0.0;
+    for (int d = 0; d < DIM; ++d) {
+      if (n_[d] > kDftMaxLen) return false;
+    }
+    sums += static_cast<double>(n_[0] * n_[1] * n_[2]) * N_[0];
+    sums += static_cast<double>(N_[0] * n_[1] * n_[2]) * N_[1];
+    if (DIM == 3) sums += static_cast<double>(N_[0] * N_[1] * n_[2]) * N_[2];
+    return sums * count_ <= kDftMaxSums && count_ * std::max({n_[2], N_[0], N_[1]}) <= 65535;
+  }
+
+  // exp(sign 2 pi i q / n_d), q < n_d, for each axis in turn.
+  void upload_dft_twiddles(int sign, hipStream_t stream,
+                           const std::shared_ptr<neonufft::Allocator>& alloc) {
+    std::vector<double2> tw;
+    for (int d = 0; d < DIM; ++d) {
+      dft_off_[d] = tw.size();
+      for (long long q = 0; q < n_[d]; ++q) {
+        const double a = 2.0 * kPi * static_cast<double>(q) / static_cast<double>(n_[d]);
+        tw.push_back(double2{std::cos(a), (sign < 0 ? -1.0 : 1.0) * std::sin(a)});
+      }
+    }
+    dft_tw_.reset(tw.size(), alloc);
+    check_hip(hipMemcpyAsync(dft_tw_.data(), tw.data(), tw.size() * sizeof(double2),
+                             hipMemcpyHostToDevice, stream),
+              "hipMemcpyAsync(twiddles)");
+    check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  }
+  const double2* dft(int d) const { return dft_tw_.data() + dft_off_[d]; }
+
   // h -> zero-padded x rows of the fine grids -> x-FFT.
   void expand_from_h(Cplx<T>* grids, hipStream_t s) {
     const long long n0 = n_[0], n1 = n_[1], n2 = n_[2], N0 = N_[0];
     const long long gstride = n0 * n1 * n2;
+    if constexpr (std::is_same_v<T, float>) {
+      if (small_) {
+        launch_dft_move(false, dft(0), h_.data(), grids, static_cast<int>(n1),
+                        static_cast<int>(n0), static_cast<int>(N0), n1, n0,
+                        static_cast<std::size_t>(count_ * n2), static_cast<int>(n2),
+                        n2 * N0 * n1, N0 * n1, gstride, n1 * n0, s);
+        return;
+      }
+    }
     launch_expand_transpose<T>(h_.data(), grids, static_cast<int>(n1), static_cast<int>(n0),
                                static_cast<int>(N0), n1, n0,
                                static_cast<std::size_t>(count_ * n2), static_cast<int>(n2),
@@ -216,9 +317,32 @@ private:
     return j;
   }
 
+  // From h on: the y-FFT; 2D then deconvolves, 3D transposes to K, runs the
+  // z-FFT and deconvolves.
   void finish_forward(T* const* fs, int order_fft, Cplx<T>* single, Cplx<T>* const* outs,
                       const IntType* st, hipStream_t s) {
     const long long n1 = n_[1], n2 = n_[2], N0 = N_[0], N1 = N_[1], N2 = N_[2];
+    if constexpr (std::is_same_v<T, float>) {
+      if (small_) {
+        if constexpr (DIM == 2) {
+          launch_dft_modes_out<2>(dft(1), h_.data(), N0 * n1, single, outs, count_,
+                                  static_cast<int>(N0), 1, static_cast<int>(n1),
+                                  static_cast<int>(N1), st[0], 0, st[1], fs[0], fs[1], fs[1],
+                                  order_fft, s);
+        } else {
+          launch_dft_move(true, dft(1), h_.data(), k_.data(), static_cast<int>(n2),
+                          static_cast<int>(n1), static_cast<int>(N1), N0 * n1, N0 * n2,
+                          static_cast<std::size_t>(count_ * N0), static_cast<int>(N0),
+                          n2 * N0 * n1, n1, N1 * N0 * n2, n2, s);
+          launch_dft_modes_out<3>(dft(2), k_.data(), N1 * N0 * n2, single, outs, count_,
+                                  static_cast<int>(N0), static_cast<int>(N1),
+                                  static_cast<int>(n2), static_cast<int>(N2), st[0], st[1], st[2],
+                                  fs[0], fs[1], fs[2], order_fft, s);
+        }
+        return;
+      }
+    }
+    py_.execute(h_.data());
     if constexpr (DIM == 2) {
       launch_modes_out<T, 2>(h_.data(), N0 * n1, single, outs, count_, static_cast<int>(N0), 1,
                              static_cast<int>(n1), static_cast<int>(N1), st[0], 0, st[1], fs[0],
@@ -240,6 +364,9 @@ private:
   int y_rows_ = 0;
   FftPlan px_, py_, pz_;
   DeviceBuffer<Cplx<T>> h_, k_;
+  bool small_ = false;  // axes transformed by sums, no FFT plans
+  DeviceBuffer<double2> dft_tw_;
+  std::size_t dft_off_[3] = {0, 0, 0};
 };
 
 }  // namespace nnf
