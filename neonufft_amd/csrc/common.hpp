@@ -214,10 +214,17 @@ struct FoldParams {
 // ES kernel evaluation parameters. For float plans the kernel is a per-piece
 // polynomial (Horner) in y = 2x - 1, fitted on the host in FP64 for the plan's
 // (ns, beta); coef[j * (deg + 1) + k] is the coefficient of y^k of piece j.
-// Double plans evaluate exp(beta (sqrt(1 - (2t/ns)^2) - 1)) directly.
+// Double plans evaluate exp(beta (sqrt(1 - (2t/ns)^2) - 1)) for the two end
+// pieces, which hold its square-root branch points, and degree-16 polynomials
+// in y for the others: pair[j * 17 + k] of piece j, 1 <= j < ns / 2 rounded up,
+// piece ns - 1 - j being its mirror image.
 constexpr int kMaxHornerCoef = 16 * 18;
+constexpr int kPairDegree = 16;
 struct EsParams {
-  float coef[kMaxHornerCoef];
+  union {
+    float coef[kMaxHornerCoef];
+    double pair[8 * (kPairDegree + 1)];
+  };
   double beta;
 };
 

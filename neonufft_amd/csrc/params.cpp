@@ -102,6 +102,31 @@ double fit_horner(int ns, double beta, int deg, double* coef) {
   return max_err;
 }
 
+void fit_pairs(int ns, double beta, double* coef) {
+  using X = long double;
+  constexpr int nc = kPairDegree + 1;
+  const X pi = 3.14159265358979323846264338327950288L;
+  X T[nc][nc] = {};  // Chebyshev polynomial T_m as monomial coefficients
+  T[0][0] = T[1][1] = 1;
+  for (int m = 2; m < nc; ++m) {
+    for (int k = 0; k < nc; ++k) T[m][k] = (k > 0 ? 2 * T[m - 1][k - 1] : X(0)) - T[m - 2][k];
+  }
+  for (int j = 1; j < (ns + 1) / 2; ++j) {
+    X f[nc], mono[nc] = {};
+    for (int k = 0; k < nc; ++k) {
+      const X t = (std::cos(pi * (k + 0.5L) / nc) + 1) / 2 + j - X(ns) / 2;
+      f[k] = std::exp(X(beta) * (std::sqrt(1 - 4 * t * t / (X(ns) * ns)) - 1));
+    }
+    for (int m = 0; m < nc; ++m) {
+      X s = 0;
+      for (int k = 0; k < nc; ++k) s += f[k] * std::cos(m * pi * (k + 0.5L) / nc);
+      s *= (m == 0 ? X(1) : X(2)) / nc;
+      for (int k = 0; k < nc; ++k) mono[k] += s * T[m][k];
+    }
+    for (int k = 0; k < nc; ++k) coef[j * nc + k] = static_cast<double>(mono[k]);
+  }
+}
+
 KernelSetup make_kernel_setup(double tol, double upsampfac, bool use_horner) {
   if (!(tol > 0.0) || !std::isfinite(tol)) throw neonufft::InputError("Neonufft:: tolerance must be positive");
   if (!(upsampfac > 1.0) || !std::isfinite(upsampfac))
@@ -115,6 +140,8 @@ KernelSetup make_kernel_setup(double tol, double upsampfac, bool use_horner) {
     std::vector<double> c(static_cast<std::size_t>(ks.ns) * (ks.horner_deg + 1));
     fit_horner(ks.ns, ks.beta, ks.horner_deg, c.data());
     for (std::size_t i = 0; i < c.size(); ++i) ks.es.coef[i] = static_cast<float>(c[i]);
+  } else {
+    fit_pairs(ks.ns, ks.beta, ks.es.pair);
   }
   const int nq = quad_nodes(ks.ns);
   std::vector<double> x(2 * nq), w(2 * nq);

@@ -38,6 +38,10 @@ KernelSetup make_kernel_setup(double tol, double upsampfac, bool use_horner);
 // y = 2x - 1; returns the max abs error over a dense check grid.
 double fit_horner(int ns, double beta, int deg, double* coef /* ns*(deg+1) */);
 
+// Inner pieces 1 <= j < (ns + 1) / 2 of the fp64 kernel (EsParams::pair), fitted
+// in extended precision by Chebyshev interpolation.
+void fit_pairs(int ns, double beta, double* coef);
+
 // Bin geometry for a grid of size n (DIM entries), element size and ns.
 // bin_override: if non-null and positive entries, used instead of the default.
 // planes: 3D fp64 defaults suit the plane kernels (planes.hip).

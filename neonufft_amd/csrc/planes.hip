@@ -14,13 +14,14 @@
 //
 // What bounds it: the matrix pipe, 64 clocks per product and SIMD; a point
 // costs 2 ns / 4 products to spread, 2 ns 4 / 16 to interpolate: 72 clocks per
-// CU at ns = 9 (counters: matrix pipe 50 % busy, the rest is the exp and sqrt
-// of the weights, 27 x 59 clocks per 64 points, which share the fp64 units).
+// CU at ns = 9. Counters at ns = 9: matrix pipe 50 % busy beside the vector
+// instructions that share the fp64 units; polynomial weights (es_device.hpp)
+// instead of exp and sqrt took spreading from 303 to 272 us.
 // The LDS-atomic kernels of spread_interp.hip pay 1458 64-bit atomics and 12
 // conversion instructions per cell there. Measured, before -> after:
-// spreading 1e6 points, 192 x 150 x 160 cells, ns = 9: 894 -> 303 us (the
+// spreading 1e6 points, 192 x 150 x 160 cells, ns = 9: 894 -> 272 us (the
 // rounding of the sums is that of fp64 FMAs); 2e6 points, 262 x 262 x 72 cells,
-// ns = 7: 775 -> 567 us; interpolation of the former ~500 -> 353 us.
+// ns = 7: 775 -> 508 us; interpolation of the former ~500 -> 340 us.
 //
 // Semantics as spread_interp.hip (reference
 // src/neonufft/gpu/kernels/spreading_kernel.cu:588-660,
@@ -76,7 +77,7 @@ __device__ inline void load_point(const PointRec<double, 3>* __restrict__ pts, u
 }
 
 // Fills the weights of a chunk of `cnt` points; mul(w) is the kz entry of
-// weight w. Wave = weight, lane = point, so every wave runs uniformly; the
+// weight w. Wave = weights, lane = point, so every wave runs uniformly; the
 // cells of kx and ky outside the kernel's window get their zeros.
 template <int NS, typename Z, typename Mul>
 __device__ __forceinline__ void fill_weights(PlaneWeights<Z>& s, double px, double py,
@@ -86,15 +87,20 @@ __device__ __forceinline__ void fill_weights(PlaneWeights<Z>& s, double px, doub
   const int p = (wave & 1) * 64 + lane;
   const int r0 = unpack_cell<3>(cell, 0), r1 = unpack_cell<3>(cell, 1);
   const int r2 = first_plane(cell);
-  for (int i = wave >> 1; i < 3 * NS; i += kPlaneWaves / 2) {
-    const int d = i / NS, j = i - d * NS;
-    const double w = es_piece<NS>(d == 0 ? px : (d == 1 ? py : pz), j, es);
+  // (axis, pair of pieces), the pairs of end pieces first: they cost the most
+  for (int i = wave >> 1; i < 3 * ((NS + 1) / 2); i += kPlaneWaves / 2) {
+    const int j = i / 3, d = i - 3 * j, j2 = NS - 1 - j;
+    double lo, hi;
+    es_pair<NS>(d == 0 ? px : (d == 1 ? py : pz), j, es, lo, hi);
     if (d == 0) {
-      s.kx[p * kPitch + r0 + j] = w;
+      s.kx[p * kPitch + r0 + j] = lo;
+      s.kx[p * kPitch + r0 + j2] = hi;
     } else if (d == 1) {
-      s.ky[p * kPitch + r1 + j] = w;
+      s.ky[p * kPitch + r1 + j] = lo;
+      s.ky[p * kPitch + r1 + j2] = hi;
     } else {
-      s.kz[p * kPitch + ((r2 + j) & 15)] = mul(w);
+      s.kz[p * kPitch + ((r2 + j) & 15)] = mul(lo);
+      s.kz[p * kPitch + ((r2 + j2) & 15)] = mul(hi);
     }
   }
   for (int i = wave >> 1; i < 2 * (16 - NS); i += kPlaneWaves / 2) {
