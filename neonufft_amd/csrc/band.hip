@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(kChunkThreads)
     row_count_kernel(const PointRec<T, 2>* __restrict__ recs, std::size_t m, BinGeom g, int ns,
                      uint32_t* __restrict__ count, uint32_t* __restrict__ rank) {
   // the records are bin-sorted: a chunk of them starts on a few dozen rows
-  chunk_rank<kChunkThreads>(m, count, rank, [&](std::size_t p) {
+  chunk_rank<kChunkThreads>(m, count, rank, 1u, [&](std::size_t p) {
     int i0x, i0y;
     rec_start(recs[p], g, ns, i0x, i0y);
     // i0y = ceil(y - ns/2) lies in [-ns/2, n1 - 1]

@@ -27,11 +27,12 @@ constexpr std::size_t kLargeChunkMin = 65536;  // items from which large chunks 
 constexpr int kChunkPerThread = 8;
 
 // Call from every thread of an NT-thread workgroup (NT a power of two),
-// grid-striding over chunks; `key_of(i)` returns a uint32_t other than
+// grid-striding over chunks; count[key * stride] counts, and `key_of(i)` returns a uint32_t other than
 // 0xFFFFFFFF.
 template <int NT, typename KeyOf>
 __device__ inline void chunk_rank(std::size_t m, uint32_t* __restrict__ count,
-                                  uint32_t* __restrict__ rank, KeyOf key_of) {
+                                  uint32_t* __restrict__ rank, uint32_t stride,
+                                  KeyOf key_of) {
   constexpr int kChunkItems = NT * kChunkPerThread;
   constexpr int kChunkSlots = 2 * kChunkItems;
   constexpr int kChunkHashBits = __builtin_ctz(kChunkSlots);
@@ -69,7 +70,7 @@ __device__ inline void chunk_rank(std::size_t m, uint32_t* __restrict__ count,
     // the chunk's range of each of its keys; the slot then holds its base
     for (int s = threadIdx.x; s < kChunkSlots; s += NT) {
       const uint32_t n = cnt[s];
-      if (n != 0) cnt[s] = atomicAdd(&count[key[s]], n);
+      if (n != 0) cnt[s] = atomicAdd(&count[static_cast<std::size_t>(key[s]) * stride], n);
     }
     __syncthreads();
 #pragma unroll

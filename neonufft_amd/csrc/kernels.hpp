@@ -31,7 +31,11 @@ constexpr uint32_t kMaxSubproblemPoints = 2048;
 // ---- points.hip: fold / rescale, counting sort by bin, subproblems -------
 template <typename TC, int DIM>
 void launch_bin_count(Loc<TC> loc, std::size_t m, const FoldParams& fp, const BinGeom& g, int ns,
-                      uint32_t* count, uint32_t* rank, hipStream_t stream);
+                      uint32_t* count, uint32_t* rank, uint32_t stride, hipStream_t stream);
+
+// dst[i] = src[i * stride], i < n.
+void launch_pick_u32(const uint32_t* src, std::size_t n, uint32_t stride, uint32_t* dst,
+                     hipStream_t stream);
 
 // TC: coordinate type read; T: precision of the point records written
 // (TC = T, or TC = double with T = float for mixed-precision type 3).

@@ -61,9 +61,24 @@ public:
     nbins_ = nbins;
     nsub_ = 0;
 
-    launch_fill_u32(t.count, nbins + 1, 0u, stream);
     launch_fill_u32(t.nsubb, nbins + 1, 0u, stream);
-    launch_bin_count<TC, DIM>(loc, m, fp, g, ns, t.count, t.rank, stream);
+    // Atomics on one cache line run one after the other, so many points over
+    // few bins count into one line per bin, in the memory of the records
+    // (written later): 1e6 points, 464 bins 50 -> 21 us. 1e7 points over 8192
+    // bins gain nothing (281 us either way).
+    constexpr uint32_t kLine = 32;
+    const bool padded = !ws && m >= 65536 && nbins <= 4096 &&
+                        nbins * kLine * sizeof(uint32_t) <= m * sizeof(PointRec<T, DIM>);
+    if (padded) {
+      uint32_t* lines = reinterpret_cast<uint32_t*>(recs_.data());
+      launch_fill_u32(lines, nbins * kLine, 0u, stream);
+      launch_bin_count<TC, DIM>(loc, m, fp, g, ns, lines, t.rank, kLine, stream);
+      launch_fill_u32(t.count + nbins, 1, 0u, stream);
+      launch_pick_u32(lines, nbins, kLine, t.count, stream);
+    } else {
+      launch_fill_u32(t.count, nbins + 1, 0u, stream);
+      launch_bin_count<TC, DIM>(loc, m, fp, g, ns, t.count, t.rank, 1u, stream);
+    }
     launch_exclusive_scan(t.count, t.start, nbins + 1, t.scan, stream);
     launch_subprob_counts(t.count, nbins, max_points, t.nsubb, stream);
     launch_exclusive_scan(t.nsubb, t.sub_start, nbins + 1, t.scan, stream);

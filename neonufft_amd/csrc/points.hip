@@ -69,8 +69,8 @@ __device__ inline uint32_t point_bin(const Loc<TC>& loc, std::size_t i, const Fo
 template <typename TC, int DIM, int NT>
 __global__ void __launch_bounds__(NT)
     bin_count_kernel(Loc<TC> loc, std::size_t m, FoldParams fp, BinGeom g, int ns,
-                     uint32_t* __restrict__ count, uint32_t* __restrict__ rank) {
-  chunk_rank<NT>(m, count, rank, [&](std::size_t i) {
+                     uint32_t* __restrict__ count, uint32_t* __restrict__ rank, uint32_t stride) {
+  chunk_rank<NT>(m, count, rank, stride, [&](std::size_t i) {
     double hx[3];
     int rel[3];
     return point_bin<TC, DIM>(loc, i, fp, g, ns, hx, rel);
@@ -181,6 +181,15 @@ __global__ void __launch_bounds__(kScanThreads)
   for (int k = 0; k < kScanItems; ++k) {
     if (base + k < n) out[base + k] = run;
     run += v[k];
+  }
+}
+
+__global__ void __launch_bounds__(kBlock)
+    pick_u32_kernel(const uint32_t* __restrict__ src, std::size_t n, uint32_t stride,
+                    uint32_t* __restrict__ dst) {
+  for (std::size_t i = threadIdx.x + static_cast<std::size_t>(blockIdx.x) * kBlock; i < n;
+       i += static_cast<std::size_t>(gridDim.x) * kBlock) {
+    dst[i] = src[i * stride];
   }
 }
 
@@ -333,16 +342,16 @@ __global__ void __launch_bounds__(kBlock)
 
 template <typename TC, int DIM>
 void launch_bin_count(Loc<TC> loc, std::size_t m, const FoldParams& fp, const BinGeom& g, int ns,
-                      uint32_t* count, uint32_t* rank, hipStream_t stream) {
+                      uint32_t* count, uint32_t* rank, uint32_t stride, hipStream_t stream) {
   if (m == 0) return;
   if (m >= kLargeChunkMin) {
     constexpr int NT = kLargeChunkThreads;
     hipLaunchKernelGGL((bin_count_kernel<TC, DIM, NT>), dim3(chunk_rank_blocks(m, NT)), dim3(NT), 0,
-                       stream, loc, m, fp, g, ns, count, rank);
+                       stream, loc, m, fp, g, ns, count, rank, stride);
   } else {
     constexpr int NT = kChunkThreads;
     hipLaunchKernelGGL((bin_count_kernel<TC, DIM, NT>), dim3(chunk_rank_blocks(m, NT)), dim3(NT), 0,
-                       stream, loc, m, fp, g, ns, count, rank);
+                       stream, loc, m, fp, g, ns, count, rank, stride);
   }
   check_launch("bin_count_kernel");
 }
@@ -386,6 +395,14 @@ void launch_exclusive_scan(const uint32_t* in, uint32_t* out, std::size_t n, uin
   hipLaunchKernelGGL(scan_tiles_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kScanThreads), 0,
                      stream, in, n, scratch, out);
   check_launch("scan_tiles_kernel");
+}
+
+void launch_pick_u32(const uint32_t* src, std::size_t n, uint32_t stride, uint32_t* dst,
+                     hipStream_t stream) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(pick_u32_kernel, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, stream, src, n,
+                     stride, dst);
+  check_launch("pick_u32_kernel");
 }
 
 void launch_fill_u32(uint32_t* p, std::size_t n, uint32_t v, hipStream_t stream) {
@@ -433,7 +450,7 @@ void launch_minmax(const T* x, std::size_t m, double* partial, hipStream_t strea
 
 #define NNF_INST_POINTS(T, DIM)                                                                 \
   template void launch_bin_count<T, DIM>(Loc<T>, std::size_t, const FoldParams&, const BinGeom&, \
-                                         int, uint32_t*, uint32_t*, hipStream_t);               \
+                                         int, uint32_t*, uint32_t*, uint32_t, hipStream_t);     \
   template void launch_bin_scatter<T, T, DIM>(Loc<T>, std::size_t, const FoldParams&,           \
                                               const BinGeom&, int, const uint32_t*,             \
                                               const uint32_t*, PointRec<T, DIM>*, uint32_t*,    \

@@ -46,24 +46,26 @@ __device__ inline void batched_copy(int total, Load load, Store store) {
   }
 }
 
-// Thread per bin: the pencils its tile meets, if it has points.
+// Thread per bin and tile plane: the pencils it meets, if the bin has points.
 template <int DIM>
 __global__ void __launch_bounds__(256)
     mark_pencils_kernel(const uint32_t* __restrict__ sub_start, BinGeom g, int ns, int rows,
                         uint32_t* __restrict__ used) {
-  const uint32_t nbins = static_cast<uint32_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2];
-  const uint32_t b = threadIdx.x + blockIdx.x * 256u;
-  if (b >= nbins || sub_start[b + 1] == sub_start[b]) return;
+  const std::size_t nbins = static_cast<std::size_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2];
+  const std::size_t i = threadIdx.x + static_cast<std::size_t>(blockIdx.x) * 256u;
+  if (i >= nbins * static_cast<unsigned>(g.tile[2])) return;
+  const uint32_t b = static_cast<uint32_t>(i / static_cast<unsigned>(g.tile[2]));
+  const int z = static_cast<int>(i % static_cast<unsigned>(g.tile[2]));
+  if (sub_start[b + 1] == sub_start[b]) return;
   const uint32_t yz = b / static_cast<uint32_t>(g.nbins[0]);
   const int oy = static_cast<int>(yz % static_cast<uint32_t>(g.nbins[1])) * g.bin[1];
   const int oz = static_cast<int>(yz / static_cast<uint32_t>(g.nbins[1])) * g.bin[2];
   const int ey = min(min(g.bin[1], g.n[1] - oy) + ns - 1, g.n[1]);
   const int ez = DIM >= 3 ? min(min(g.bin[2], g.n[2] - oz) + ns - 1, g.n[2]) : 1;
   const int groups = (g.n[1] + rows - 1) / rows;
-  for (int z = 0; z < ez; ++z) {
-    const int gz = DIM >= 3 ? wrap_once(oz - ns / 2 + z, g.n[2]) : 0;
-    for (int y = 0; y < ey; ++y) used[gz * groups + wrap_once(oy - ns / 2 + y, g.n[1]) / rows] = 1u;
-  }
+  if (z >= ez) return;
+  const int gz = DIM >= 3 ? wrap_once(oz - ns / 2 + z, g.n[2]) : 0;
+  for (int y = 0; y < ey; ++y) used[gz * groups + wrap_once(oy - ns / 2 + y, g.n[1]) / rows] = 1u;
 }
 
 // True when the pencil of this workgroup meets no tile (uniform).
@@ -665,8 +667,9 @@ void launch_expand_rows_ifft(const RowFftJob<T>& job, hipStream_t stream) {
 template <int DIM>
 void launch_mark_pencils(const uint32_t* sub_start, const BinGeom& g, int ns, int rows,
                          uint32_t* used, hipStream_t stream) {
-  const std::size_t nbins = static_cast<std::size_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2];
-  hipLaunchKernelGGL((mark_pencils_kernel<DIM>), dim3(static_cast<unsigned>((nbins + 255) / 256)),
+  const std::size_t items =
+      static_cast<std::size_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2] * static_cast<unsigned>(g.tile[2]);
+  hipLaunchKernelGGL((mark_pencils_kernel<DIM>), dim3(static_cast<unsigned>((items + 255) / 256)),
                      dim3(256), 0, stream, sub_start, g, ns, rows, used);
   check_launch("mark_pencils_kernel");
 }
