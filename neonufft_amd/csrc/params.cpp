@@ -106,6 +106,8 @@ void fit_pairs(int ns, double beta, double* coef) {
   using X = long double;
   constexpr int nc = kPairDegree + 1;
   const X pi = 3.14159265358979323846264338327950288L;
+  X wave[4 * nc];  // cos(pi q / (2 nc)): the angles m (k + 1/2) pi / nc
+  for (int q = 0; q < 4 * nc; ++q) wave[q] = std::cos(pi * q / (2 * nc));
   X T[nc][nc] = {};  // Chebyshev polynomial T_m as monomial coefficients
   T[0][0] = T[1][1] = 1;
   for (int m = 2; m < nc; ++m) {
@@ -114,12 +116,12 @@ void fit_pairs(int ns, double beta, double* coef) {
   for (int j = 1; j < (ns + 1) / 2; ++j) {
     X f[nc], mono[nc] = {};
     for (int k = 0; k < nc; ++k) {
-      const X t = (std::cos(pi * (k + 0.5L) / nc) + 1) / 2 + j - X(ns) / 2;
+      const X t = (wave[2 * k + 1] + 1) / 2 + j - X(ns) / 2;
       f[k] = std::exp(X(beta) * (std::sqrt(1 - 4 * t * t / (X(ns) * ns)) - 1));
     }
     for (int m = 0; m < nc; ++m) {
       X s = 0;
-      for (int k = 0; k < nc; ++k) s += f[k] * std::cos(m * pi * (k + 0.5L) / nc);
+      for (int k = 0; k < nc; ++k) s += f[k] * wave[m * (2 * k + 1) % (4 * nc)];
       s *= (m == 0 ? X(1) : X(2)) / nc;
       for (int k = 0; k < nc; ++k) mono[k] += s * T[m][k];
     }
