@@ -218,7 +218,7 @@ typedef struct nnf_plan_info {
   int64_t num_subproblems;
   int64_t num_points;
   int64_t num_out_points;/* type 3 targets */
-  int horner_degree;     /* fp32 ES polynomial degree (0 = exact exp/sqrt) */
+  int horner_degree;     /* fp32 ES polynomial degree (0 in fp64) */
   int quad_nodes;        /* Gauss-Legendre nodes on (0,1) for phihat */
   int spread_mode;       /* type-1 spreading: NNF_SPREAD_TILES, _BANDS (fused x-FFT) or _BANDS_GRID */
   int band_rows;         /* fine-grid rows per band (row bands), else 0 */

@@ -13,7 +13,9 @@
 //    the grid (no global atomics, fixed summation order); interpolation
 //    loads the tile once with coalesced reads and gathers from LDS;
 //  - kernel weights come from per-piece Horner polynomials in registers (fp32)
-//    or the exact exp/sqrt formula (fp64);
+//    or, in fp64, from the exp/sqrt formula at the kernel's ends and
+//    polynomials between (es_device.hpp);
+//  - 3D fp64 with tiles of at most 16 x 16 cells in x and y goes to planes.hip;
 //  - subproblem -> workgroup mapping keeps neighbouring bins on one XCD.
 #include "es_device.hpp"
 
