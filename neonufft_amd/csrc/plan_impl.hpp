@@ -679,10 +679,11 @@ public:
     // interpolation at 0.024, where groups of 16 points are half empty.
     std::size_t cells = 1;
     for (int d = 0; d < DIM; ++d) cells *= static_cast<std::size_t>(gi_.fft_grid_size[d]);
-    geom_out_ = choose_bins(DIM, gi_.fft_grid_size, ks_.ns, sizeof(Cplx<T>), tune_.bin,
-                            static_cast<std::size_t>(num_out) >= cells / 10);
-    out_pts_.build(l, static_cast<std::size_t>(num_out), fp, geom_out_, ks_.ns, tune_.max_points,
+    const BinGeom geom = choose_bins(DIM, gi_.fft_grid_size, ks_.ns, sizeof(Cplx<T>), tune_.bin,
+                                     static_cast<std::size_t>(num_out) >= cells / 10);
+    out_pts_.build(l, static_cast<std::size_t>(num_out), fp, geom, ks_.ns, tune_.max_points,
                    stream_, alloc_);
+    geom_out_ = geom;  // of the points held: a refused call keeps points and bins together
     post_.ensure(num_out ? static_cast<std::size_t>(num_out) : 1, alloc_);
     launch_postphase<TC, T, DIM>(sign_, l, out_pts_.perm(), static_cast<std::size_t>(num_out),
                                  gi_.input_offsets, gi_.output_offsets, scale, ks_.quad,
