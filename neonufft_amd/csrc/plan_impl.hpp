@@ -365,13 +365,14 @@ public:
   void transform_type_1(const Cplx<T>* in, Cplx<T>* out, const IntType* out_strides) {
     require_points();
     if (!out || !out_strides) throw neonufft::InputError("Neonufft:: null output");
+    if (pts_.size() && !in) throw neonufft::InputError("Neonufft:: null input");
+    // nothing refuses the call from here on
     grid_partial_ = false;  // the grid is work memory again, h is overwritten
     T* fs[3] = {fs_[0].data(), fs_[1].data(), fs_[2].data()};
     if constexpr (DIM == 2) {
       if (bands_on_ && band_.fft) {
         // gather, then spread + x-FFT per band straight into the pruned
         // FFT's intermediate; y-FFT and deconvolution follow
-        if (pts_.size() && !in) throw neonufft::InputError("Neonufft:: null input");
         launch_clear_bounds(bounds_.data(), bounds_.size(), stream_);
         launch_band_gather<T>(nullptr, band_job(in), 1, pts_.size(), stream_);
         const int nb = static_cast<int>((n_[1] + band_rows_ - 1) / band_rows_);
