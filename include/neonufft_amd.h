@@ -236,13 +236,14 @@ int nnf_plan_spread(nnf_plan plan, const void* in, int accumulate);
 int nnf_plan_spread_tiles(nnf_plan plan, const void* in);
 /* The tile reduction alone: fine grid (+)= sum of the covering tiles. */
 int nnf_plan_reduce_tiles(nnf_plan plan, int accumulate);
-/* Interpolate the current fine grid at the plan's points into `out`
- * (type-2 stage 3). */
+/* Interpolate the current fine grid (see nnf_plan_fine_grid) at the plan's
+ * points into `out` (type-2 stage 3). */
 int nnf_plan_interp(nnf_plan plan, void* out);
 /* Device pointer of the plan's fine grid (n_0 x n_1 x n_2 complex, x fastest).
  * It holds the last spread's sums or the last type 2's fine-grid values; a
  * type 1 leaves it unspecified. Until a plan is asked for it, type 2 forms the
- * rows that the plan's points read, and completes the grid when asked. */
+ * rows that the plan's points read, and completes the grid when asked; from
+ * then on it forms every row, also in HIP graphs captured before. */
 int nnf_plan_fine_grid(nnf_plan plan, void** grid);
 /* Device pointer of the deconvolution factors fs_d[0..n_d/2] (T). */
 int nnf_plan_fseries(nnf_plan plan, int d, const void** fs);

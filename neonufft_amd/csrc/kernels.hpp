@@ -312,10 +312,14 @@ struct RowFftJob {
   const Cplx<T>* tw;          // twiddles as for the row bands (tw[N/2 + q])
   int N0, log2n0, rows, log2rows, pitch;
   // One word per pencil, z * ceil(n1 / rows) + y / rows: non-zero where the
-  // tile of a bin with points meets it; null = every pencil counts.
+  // tile of a bin with points meets it; null = every pencil counts. The word
+  // after the last pencil is non-zero once type 2 has to form every row.
   const uint32_t* used;
+  // One word per pencil: zero where the grid lacks the rows that type 2 left
+  // out, which h still holds.
+  uint32_t* formed;
 };
-// used[pencil] = 1 for the pencils above; `used` is zero beforehand.
+// used[pencil] = 1 for the pencils above; their words are zero beforehand.
 template <int DIM>
 void launch_mark_pencils(const uint32_t* sub_start, const BinGeom& g, int ns, int rows,
                          uint32_t* used, hipStream_t stream);
@@ -334,6 +338,9 @@ void launch_reduce_rows_fft(const RowFftJob<T>& job, int ns, hipStream_t stream)
 // Type 2: h -> fine grid.
 template <typename T>
 void launch_expand_rows_ifft(const RowFftJob<T>& job, hipStream_t stream);
+// ... of the pencils that are not formed yet.
+template <typename T>
+void launch_form_missing_rows(const RowFftJob<T>& job, hipStream_t stream);
 
 // ---- rows.hip: the y and z passes of a 3D pruned FFT in LDS --------------
 // For power-of-two n1, n2 >= 32. Between h[(z N0 + x') n1 + y] and

@@ -191,7 +191,10 @@ public:
       if (row_rows_ > 0) {
         pencils_ = static_cast<std::size_t>((n_[1] + row_rows_ - 1) / row_rows_) *
                    static_cast<std::size_t>(n_[2]);
-        used_.reset(pencils_, alloc_);
+        used_.reset(pencils_ + 1, alloc_);
+        formed_.reset(pencils_, alloc_);
+        launch_fill_u32(used_.data() + pencils_, 1, 0u, stream_);
+        launch_fill_u32(formed_.data(), pencils_, 1u, stream_);
       }
     }
     // 3D with the row kernels: the y and z passes in LDS too, when both
@@ -332,8 +335,11 @@ public:
   }
   void reduce_tiles(bool accumulate) {
     require_points();
-    if (accumulate) complete_grid();
-    grid_partial_ = false;
+    if (accumulate) {
+      complete_grid();
+    } else {
+      grid_overwritten();
+    }
     if constexpr (DIM == 2) {
       if (bands_on_) {
         const int nb = static_cast<int>((n_[1] + band_rows_ - 1) / band_rows_);
@@ -366,13 +372,14 @@ public:
     require_points();
     if (!out || !out_strides) throw neonufft::InputError("Neonufft:: null output");
     if (pts_.size() && !in) throw neonufft::InputError("Neonufft:: null input");
-    // nothing refuses the call from here on
-    grid_partial_ = false;  // the grid is work memory again, h is overwritten
+    // Nothing refuses the call from here on. The grid is work memory again, and
+    // h is overwritten (the row kernels note it themselves).
     T* fs[3] = {fs_[0].data(), fs_[1].data(), fs_[2].data()};
     if constexpr (DIM == 2) {
       if (bands_on_ && band_.fft) {
         // gather, then spread + x-FFT per band straight into the pruned
         // FFT's intermediate; y-FFT and deconvolution follow
+        grid_overwritten();
         launch_clear_bounds(bounds_.data(), bounds_.size(), stream_);
         launch_band_gather<T>(nullptr, band_job(in), 1, pts_.size(), stream_);
         const int nb = static_cast<int>((n_[1] + band_rows_ - 1) / band_rows_);
@@ -389,6 +396,7 @@ public:
         // tiles -> retained x modes in one pass, then the remaining passes
         spread_tiles(in);
         launch_reduce_rows_fft<T, DIM>(row_job(used_.data()), ks_.ns, stream_);
+        grid_partial_ = false;
         if (axis_rows_y_ > 0) {
           launch_axis_fft_type1<T>(axis_job(out, nullptr, out_strides), stream_);
         } else {
@@ -426,6 +434,7 @@ public:
         // only the rows that points read, unless the caller has asked for the grid
         launch_expand_rows_ifft<T>(row_job(grid_shown_ ? nullptr : used_.data()), stream_);
         grid_partial_ = !grid_shown_;
+        note_capture();
       } else {
         pfft_.backward(in, nullptr, in_strides, fs, order_fft(), grid_.data(), stream_);
       }
@@ -454,9 +463,13 @@ public:
     info->band_rows = bands_on_ ? band_rows_ : 0;
   }
 
-  // From here on type 2 forms every row of the grid: the caller may read it.
+  // From here on type 2 forms every row of the grid, also in graphs captured
+  // before: the caller may read it.
   Cplx<T>* fine_grid() {
     complete_grid();
+    if (row_rows_ > 0 && !grid_shown_) {
+      launch_fill_u32(used_.data() + pencils_, 1, 1u, stream_);
+    }
     grid_shown_ = true;
     return grid_.data();
   }
@@ -507,17 +520,42 @@ private:
     return j;
   }
 
+  // Whether the grid lacks rows is kept per pencil on the device (formed_), where
+  // replayed graphs keep it too. grid_partial_ spares the calls that would find
+  // nothing to do; it follows eager calls only, so nothing is spared once a
+  // call of the plan has been captured.
+  void note_capture() {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream_, &status) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    captured_ = captured_ || status != hipStreamCaptureStatusNone;
+  }
+  bool may_lack_rows() {
+    if (row_rows_ == 0) return false;
+    note_capture();
+    return grid_partial_ || captured_;
+  }
+
   // The rows that the last type 2 left out, from the h it left behind.
   void complete_grid() {
     if constexpr (DIM >= 2) {
-      if (grid_partial_) launch_expand_rows_ifft<T>(row_job(nullptr), stream_);
+      if (may_lack_rows()) launch_form_missing_rows<T>(row_job(nullptr), stream_);
     }
+    grid_partial_ = false;
+  }
+
+  // The grid or h is about to be overwritten: no row is missing any more.
+  void grid_overwritten() {
+    if (may_lack_rows()) launch_fill_u32(formed_.data(), pencils_, 1u, stream_);
     grid_partial_ = false;
   }
 
   RowFftJob<T> row_job(const uint32_t* used) const {
     RowFftJob<T> j{};
     j.used = used;
+    j.formed = formed_.data();
     j.tiles = tiles_.data();
     j.sub_start = pts_.sub_starts();
     j.g = geom_;
@@ -577,7 +615,9 @@ private:
   bool bands_on_ = false;         // row bands used for the current points
   std::size_t pencils_ = 0;       // pencils of the row kernels
   DeviceBuffer<uint32_t> used_;   // pencils that the tiles of the points meet
-  bool grid_partial_ = false;     // the grid lacks the rows no point reads
+  DeviceBuffer<uint32_t> formed_;  // pencils whose rows the grid holds
+  bool grid_partial_ = false;     // the grid may lack the rows no point reads
+  bool captured_ = false;         // ... or after any replay
   bool grid_shown_ = false;       // fine_grid() has handed out the grid
   bool points_valid_ = false;     // the last set_points succeeded
   std::vector<uint32_t> row_host_;  // row offsets of the view (balance check)

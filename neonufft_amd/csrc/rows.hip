@@ -68,11 +68,11 @@ __global__ void __launch_bounds__(256)
   for (int y = 0; y < ey; ++y) used[gz * groups + wrap_once(oy - ns / 2 + y, g.n[1]) / rows] = 1u;
 }
 
-// True when the pencil of this workgroup meets no tile (uniform).
+// Word of a pencil in used[] and formed[].
 template <typename T>
-__device__ inline bool pencil_unused(const RowFftJob<T>& job, int z, int y0) {
+__device__ inline int pencil_word(const RowFftJob<T>& job, int z, int y0) {
   const int groups = (job.g.n[1] + job.rows - 1) / job.rows;
-  return job.used && job.used[z * groups + (y0 >> job.log2rows)] == 0u;
+  return z * groups + (y0 >> job.log2rows);
 }
 
 // Pencil of workgroup blockIdx.x: rows [y0, y0 + rk) of plane z. Pencils
@@ -100,7 +100,10 @@ __global__ void __launch_bounds__(kRowThreads<T>)
   const BinGeom& g = job.g;
   const int n0 = g.n[0], n1 = g.n[1];
   const Pencil pc = pencil_of(job.rows, n1);
-  if (pencil_unused(job, pc.z, pc.y0)) {
+  const int word = pencil_word(job, pc.z, pc.y0);
+  // h no longer holds the modes of rows that type 2 left out
+  if (threadIdx.x == 0) job.formed[word] = 1u;
+  if (job.used[word] == 0u) {
     // no tile: its rows and their modes are zero
     Cplx<T>* __restrict__ hz = job.h + static_cast<std::size_t>(pc.z) * job.N0 * n1 + pc.y0;
     for (int i = threadIdx.x; i < (job.N0 << job.log2rows); i += NT) {
@@ -302,17 +305,29 @@ __global__ void __launch_bounds__(kRowThreads<T>)
   }
 }
 
-template <typename T>
+// MISSING: the pencils that are not formed yet; else those in use, noting for
+// every pencil whether it was formed. The notes are in device memory, so they
+// also follow calls that a graph replays.
+template <typename T, bool MISSING>
 __global__ void __launch_bounds__(kRowThreads<T>) expand_rows_ifft_kernel(RowFftJob<T> job) {
   constexpr int NT = kRowThreads<T>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int n0 = job.g.n[0], n1 = job.g.n[1];
   const Pencil pc = pencil_of(job.rows, n1);
-  if (pencil_unused(job, pc.z, pc.y0)) return;  // no point reads its rows
+  const int word = pencil_word(job, pc.z, pc.y0);
+  if constexpr (MISSING) {
+    if (job.formed[word] != 0u) return;
+  } else {
+    const int all = ((n1 + job.rows - 1) / job.rows) * job.g.n[2];
+    const bool form = !job.used || job.used[word] != 0u || job.used[all] != 0u;
+    if (threadIdx.x == 0) job.formed[word] = form ? 1u : 0u;
+    if (!form) return;  // no point reads its rows
+  }
   T* fre = reinterpret_cast<T*>(smem_raw);
   T* fim = fre + job.rows * job.pitch;
   for (int i = threadIdx.x; i < 2 * job.rows * job.pitch; i += NT) fre[i] = T(0);
   __syncthreads();
+  if (MISSING && threadIdx.x == 0) job.formed[word] = 1u;  // (every lane has read it)
   // retained x modes of the pencil's rows at their fine positions
   const int N0 = job.N0;
   const int P = N0 - N0 / 2;
@@ -654,14 +669,24 @@ void launch_reduce_rows_fft(const RowFftJob<T>& job, int ns, hipStream_t stream)
   check_launch("reduce_rows_fft_kernel");
 }
 
-template <typename T>
-void launch_expand_rows_ifft(const RowFftJob<T>& job, hipStream_t stream) {
+template <typename T, bool MISSING>
+void launch_expand(const RowFftJob<T>& job, hipStream_t stream) {
   const int groups = (job.g.n[1] + job.rows - 1) / job.rows;
   const std::size_t blocks = static_cast<std::size_t>(groups) * job.g.n[2];
   const std::size_t lds = row_fft_lds_bytes(job.rows, job.pitch, sizeof(T), 0);
-  hipLaunchKernelGGL((expand_rows_ifft_kernel<T>), dim3(static_cast<unsigned>(blocks)),
+  hipLaunchKernelGGL((expand_rows_ifft_kernel<T, MISSING>), dim3(static_cast<unsigned>(blocks)),
                      dim3(kRowThreads<T>), lds, stream, job);
   check_launch("expand_rows_ifft_kernel");
+}
+
+template <typename T>
+void launch_expand_rows_ifft(const RowFftJob<T>& job, hipStream_t stream) {
+  launch_expand<T, false>(job, stream);
+}
+
+template <typename T>
+void launch_form_missing_rows(const RowFftJob<T>& job, hipStream_t stream) {
+  launch_expand<T, true>(job, stream);
 }
 
 template <int DIM>
@@ -684,6 +709,8 @@ template void launch_reduce_rows_fft<double, 2>(const RowFftJob<double>&, int, h
 template void launch_reduce_rows_fft<double, 3>(const RowFftJob<double>&, int, hipStream_t);
 template void launch_expand_rows_ifft<float>(const RowFftJob<float>&, hipStream_t);
 template void launch_expand_rows_ifft<double>(const RowFftJob<double>&, hipStream_t);
+template void launch_form_missing_rows<float>(const RowFftJob<float>&, hipStream_t);
+template void launch_form_missing_rows<double>(const RowFftJob<double>&, hipStream_t);
 
 template <typename T>
 void launch_axis_fft_type1(const AxisFftJob<T>& job, hipStream_t stream) {

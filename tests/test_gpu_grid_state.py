@@ -77,3 +77,24 @@ def test_refused_type_1_leaves_the_grid(modes):
     p.interp(out)
     torch.cuda.synchronize()
     assert rel(out.cpu().numpy(), v.at_y(v.f)) < BOUND
+
+
+@pytest.mark.parametrize("modes", SHAPES)
+def test_accumulating_spread_and_the_grid_after_type_2(modes):
+    v = Inputs(modes)
+    p = v.plan(v.dx)
+    v.stale(p)
+    p.transform_type_2(v.df, None, v.out())
+    p.spread(v.dc, accumulate=True)
+    cells = int(np.prod(p.info()["grid"]))
+    got = d2h(p.fine_grid_ptr(), cells, np.complex64)
+    ref = v.plan(v.dx)
+    ref.spread(v.dc)
+    sums = d2h(ref.fine_grid_ptr(), cells, np.complex64)
+    want = v.whole_grid(v.df).astype(np.complex128) + sums
+    assert rel(got, want) < 1e-6  # the same kernels: one rounding of the sum
+    # asked for at once
+    p = v.plan(v.dx)
+    v.stale(p)
+    p.transform_type_2(v.df, None, v.out())
+    assert rel(d2h(p.fine_grid_ptr(), cells, np.complex64), v.whole_grid(v.df)) < 1e-6
