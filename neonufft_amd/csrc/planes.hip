@@ -5,27 +5,31 @@
 // T_z[y][x] += sum_p (ky[p][y] kz[p][z] c_p) kx[p][x]: one v_mfma_f64_16x16x4
 // per component and 4 points, the kernel weights padded to the 16-cell window
 // by zeros. Interpolation contracts the same way:
-// V_z[x][p] = sum_y G_z[y][x] (ky[p][y] kz[p][z]), 4 products per plane,
+// V[x][p] = sum_z sum_y G_z[y][x] (ky[p][y] kz[p][z]), 4 products per plane,
 // component and 16 points, then a dot with kx[p].
 // A subproblem's points are ordered by their first kernel plane
 // (launch_plane_order), so the points that touch a plane are a range, and the
-// planes of a subproblem are finished in order. Each wave keeps two planes in
-// registers; no tile is held in LDS, which carries the weights only.
+// planes of a subproblem are finished in order. In spreading each wave keeps two
+// planes in registers; no tile is held in LDS, which carries the weights only.
 //
 // What bounds it: the matrix pipe, 64 clocks per product and SIMD; a point
 // costs 2 ns / 4 products to spread, 2 ns 4 / 16 to interpolate: 72 clocks per
-// CU at ns = 9. Counters at ns = 9: matrix pipe 50 % busy beside the vector
-// instructions that share the fp64 units; polynomial weights (es_device.hpp)
-// instead of exp and sqrt took spreading from 303 to 272 us.
+// CU at ns = 9. Counters at ns = 9: matrix pipe 50 % busy (both directions)
+// beside the vector instructions that share the fp64 units; polynomial weights
+// (es_device.hpp) instead of exp and sqrt took spreading from 303 to 272 us.
 // The LDS-atomic kernels of spread_interp.hip pay 1458 64-bit atomics and 12
 // conversion instructions per cell there. Measured, before -> after:
 // spreading 1e6 points, 192 x 150 x 160 cells, ns = 9: 894 -> 272 us (the
 // rounding of the sums is that of fp64 FMAs); 2e6 points, 262 x 262 x 72 cells,
-// ns = 7: 775 -> 508 us; interpolation of the former ~500 -> 340 us.
+// ns = 7: 775 -> 508 us. Interpolation, LDS kernel -> planes, 128^3 cells: ns = 9,
+// 0.02 / 0.2 / 2 points per cell 218 / 223 / 1038 -> 42 / 133 / 872 us; ns = 12
+// 940 / 960 / 2594 -> 92 / 168 / 1156 us; ns = 7 86 / 111 / 600 -> 29 / 101 / 717 us.
 //
 // Semantics as spread_interp.hip (reference
 // src/neonufft/gpu/kernels/spreading_kernel.cu:588-660,
 // interpolation_kernel.cu:193-319).
+#include <algorithm>
+
 #include "es_device.hpp"
 
 namespace nnf {
@@ -44,14 +48,13 @@ constexpr int kPlaneRows = kPlaneChunk + 16;
 __device__ inline int first_plane(uint32_t cell) { return unpack_cell<3>(cell, 2); }
 
 // Kernel weights of a chunk of points. kx and ky are dense over the tile's 16
-// cells; kz[p][z & 15] holds the NS planes of point p only (spreading: times
-// the point's strength), the other entries are stale. zs[z] = points of the
+// cells; kz[p][z & 15] holds the NS planes of point p only, times the point's
+// strength, the other entries are stale. zs[z] = points of the
 // chunk that start below plane z; planes below zlast receive nothing from
 // later chunks.
-template <typename Z>
 struct PlaneWeights {
   double kx[kPlaneRows * kPitch], ky[kPlaneRows * kPitch];
-  Z kz[kPlaneRows * kPitch];
+  Cplx<double> kz[kPlaneRows * kPitch];
   int zs[kMaxTilePlanes + 1];
   int zlast;
 };
@@ -76,14 +79,13 @@ __device__ inline void load_point(const PointRec<double, 3>* __restrict__ pts, u
   before = pts[max(p, begin + 1) - 1].cell;
 }
 
-// Fills the weights of a chunk of `cnt` points; mul(w) is the kz entry of
-// weight w. Wave = weights, lane = point, so every wave runs uniformly; the
+// Fills the weights of a chunk of `cnt` points of strengths c. Wave = weights, lane = point, so every wave runs uniformly; the
 // cells of kx and ky outside the kernel's window get their zeros.
-template <int NS, typename Z, typename Mul>
-__device__ __forceinline__ void fill_weights(PlaneWeights<Z>& s, double px, double py,
-                                             double pz, uint32_t cell, uint32_t before, int cnt,
-                                             int planes, int wave, int lane, const EsParams& es,
-                                             Mul mul) {
+template <int NS>
+__device__ __forceinline__ void fill_weights(PlaneWeights& s, double px, double py, double pz,
+                                             const Cplx<double>& c, uint32_t cell, uint32_t before,
+                                             int cnt, int planes, int wave, int lane,
+                                             const EsParams& es) {
   const int p = (wave & 1) * 64 + lane;
   const int r0 = unpack_cell<3>(cell, 0), r1 = unpack_cell<3>(cell, 1);
   const int r2 = first_plane(cell);
@@ -99,8 +101,8 @@ __device__ __forceinline__ void fill_weights(PlaneWeights<Z>& s, double px, doub
       s.ky[p * kPitch + r1 + j] = lo;
       s.ky[p * kPitch + r1 + j2] = hi;
     } else {
-      s.kz[p * kPitch + ((r2 + j) & 15)] = mul(lo);
-      s.kz[p * kPitch + ((r2 + j2) & 15)] = mul(hi);
+      s.kz[p * kPitch + ((r2 + j) & 15)] = Cplx<double>{lo * c.x, lo * c.y};
+      s.kz[p * kPitch + ((r2 + j2) & 15)] = Cplx<double>{hi * c.x, hi * c.y};
     }
   }
   for (int i = wave >> 1; i < 2 * (16 - NS); i += kPlaneWaves / 2) {
@@ -125,7 +127,7 @@ __device__ __forceinline__ void fill_weights(PlaneWeights<Z>& s, double px, doub
 template <int NS>
 __device__ __forceinline__ void plane_spread(const SpreadJob<double, 3>& job, const Subprob& sp,
                                              uint32_t sidx, const EsParams& es) {
-  __shared__ PlaneWeights<Cplx<double>> s;
+  __shared__ PlaneWeights s;
   const BinGeom& g = job.g;
   const int t0 = g.tile[0], t1 = g.tile[1], t2 = g.tile[2];
   const int lane = threadIdx.x & 63;
@@ -151,8 +153,7 @@ __device__ __forceinline__ void plane_spread(const SpreadJob<double, 3>& job, co
   Cplx<double> c = load_strength(p);
   for (uint32_t base = 0; base < sp.count; base += kPlaneChunk) {
     const int cnt = static_cast<int>(min(static_cast<uint32_t>(kPlaneChunk), sp.count - base));
-    fill_weights<NS>(s, px, py, pz, cell, before, cnt, g.bin[2], wave, lane, es,
-                     [&](double w) { return Cplx<double>{w * c.x, w * c.y}; });
+    fill_weights<NS>(s, px, py, pz, c, cell, before, cnt, g.bin[2], wave, lane, es);
     __syncthreads();
     const bool last = base + kPlaneChunk >= sp.count;
     if (!last) {
@@ -228,17 +229,27 @@ __global__ void __launch_bounds__(kPlaneThreads, 4)
   plane_spread<NS>(job, sp, sidx, es);
 }
 
-// Interpolation: the same sweep with the wave's planes of the grid as the
-// operand held in registers. part[w][p] = the planes of wave w.
+// Interpolation. A wave takes 16 points in plane order and sums over all the
+// planes they touch in the accumulators, so that the dot with kx and the sums
+// across lanes are paid once per 16 points, and waves depend on no other wave.
+// The planes come from the caches: neighbouring waves take neighbouring
+// points, hence the same planes.
+constexpr int kInterpWaves = 4;
+constexpr int kInterpThreads = 64 * kInterpWaves;
+constexpr int kInterpTake = 32;  // points whose weights a wave holds at a time
+
 template <int NS>
 __device__ __forceinline__ void plane_interp(const InterpJob<double, 3>& job, const Subprob& sp,
                                              const EsParams& es) {
-  __shared__ PlaneWeights<double> s;
-  __shared__ Cplx<double> part[kPlaneWaves][kPlaneChunk];
+  constexpr int kP = NS | 1;  // weights of one point and axis, odd pitch
+  __shared__ double weights[kInterpWaves][3][kInterpTake * kP];
   const BinGeom& g = job.g;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int li = lane & 15, lk = lane >> 4;
+  double* kx = weights[wave][0];
+  double* ky = weights[wave][1];
+  double* kz = weights[wave][2];
 
   int org[3], ext[3];
   {
@@ -251,119 +262,121 @@ __device__ __forceinline__ void plane_interp(const InterpJob<double, 3>& job, co
       ext[d] = min(g.bin[d], g.n[d] - o) + NS - 1;
     }
   }
-  // Lane holds cells (x = li, y = 4 i + lk) of a plane. Cells past the bin's
+  // Lane holds cells (x = li, y = 4 q + lk) of a plane. Cells past the bin's
   // extent repeat its edge: their weights are zero.
   const int gx = wrap_once(org[0] + min(li, ext[0] - 1), g.n[0]);
   std::size_t row[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gy = wrap_once(org[1] + min(4 * i + lk, ext[1] - 1), g.n[1]);
-    row[i] = static_cast<std::size_t>(gx) +
+  for (int q = 0; q < 4; ++q) {
+    const int gy = wrap_once(org[1] + min(4 * q + lk, ext[1] - 1), g.n[1]);
+    row[q] = static_cast<std::size_t>(gx) +
              static_cast<std::size_t>(g.n[0]) * static_cast<std::size_t>(gy);
   }
   const std::size_t area = static_cast<std::size_t>(g.n[0]) * static_cast<std::size_t>(g.n[1]);
-  Cplx<double> v[2][4];
-  int plane[2] = {wave, wave + kPlaneWaves};
-  auto load_plane = [&](int k) __attribute__((always_inline)) {
-    if (plane[k] < ext[2]) {
-      const Cplx<double>* src =
-          job.grid + area * static_cast<std::size_t>(wrap_once(org[2] + plane[k], g.n[2]));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[k][i] = src[row[i]];
-    }
+  auto plane_at = [&](int z) {
+    return job.grid + area * static_cast<std::size_t>(wrap_once(org[2] + z, g.n[2]));
   };
-  // nothing of the subproblem lies below its first point's first plane
-  const int z0 = __builtin_amdgcn_readfirstlane(first_plane(job.pts[sp.begin].cell));
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    if (plane[k] < z0) plane[k] += (z0 - plane[k] + 2 * kPlaneWaves - 1) & ~(2 * kPlaneWaves - 1);
-    load_plane(k);
-  }
 
-  double px, py, pz;
-  uint32_t cell, before;
-  load_point(job.pts, chunk_point(sp, 0, wave, lane), sp.begin, px, py, pz, cell, before);
-  for (uint32_t base = 0; base < sp.count; base += kPlaneChunk) {
-    const int cnt = static_cast<int>(min(static_cast<uint32_t>(kPlaneChunk), sp.count - base));
-    fill_weights<NS>(s, px, py, pz, cell, before, cnt, g.bin[2], wave, lane, es, [](double w) { return w; });
-    for (int i = lane; i < kPlaneChunk; i += 64) part[wave][i] = Cplx<double>{0.0, 0.0};
-    __syncthreads();
-    const bool last = base + kPlaneChunk >= sp.count;
-    if (!last) {
-      load_point(job.pts, chunk_point(sp, base + kPlaneChunk, wave, lane), sp.begin, px, py, pz,
-                 cell, before);
-    }
-    const int zlast = __builtin_amdgcn_readfirstlane(s.zlast);
-    // the two planes in turn, so that one's successor loads behind the other
-    bool open[2] = {plane[0] < ext[2], plane[1] < ext[2]};
-    while (open[0] || open[1]) {
+  // 16 or 32 points per wave and round, so that few points use every wave
+  const uint32_t take = sp.count > 16 * kInterpWaves ? kInterpTake : 16;
+  for (uint32_t base = wave * take; base < sp.count; base += kInterpWaves * take) {
+    const int cnt = static_cast<int>(min(take, sp.count - base));
+    // two lanes per point: one forms the weights of x, one those of y, both z
+    const int own = lane & (kInterpTake - 1);
+    const uint32_t mine = sp.begin + base + static_cast<uint32_t>(min(own, cnt - 1));
+    const PointRec<double, 3> rec = job.pts[mine];
+    const uint32_t to = job.perm[mine];
+    const bool second = lane >= kInterpTake;
+    const double x = second ? rec.x[1] : rec.x[0];
+    double* w = (second ? ky : kx) + own * kP;
+#pragma unroll 1
+    for (int j = 0; j < (NS + 1) / 2; ++j) es_pair<NS>(x, j, es, w[j], w[NS - 1 - j]);
+    w = kz + own * kP;
+    const int end = second ? NS - 1 : 0;  // z: an end piece each
+    w[end] = es_exact<NS>(rec.x[2], end, es);
+#pragma unroll 1
+    for (int j = 1; j < (NS + 1) / 2; ++j) es_pair<NS>(rec.x[2], j, es, w[j], w[NS - 1 - j]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    for (int first = 0; first < cnt; first += 16) {
+      const int i = first + li;  // this lane's point
+      const bool in = i < cnt;
+      const uint32_t cell = __shfl(rec.cell, i, 64);
+      const int r0 = unpack_cell<3>(cell, 0), r1 = unpack_cell<3>(cell, 1);
+      const int r2 = first_plane(cell);
+      const int zbeg = __builtin_amdgcn_readlane(r2, 0);
+      const int zend = __builtin_amdgcn_readlane(r2, min(15, cnt - 1 - first)) + NS;
+      double wy[4];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (!open[k]) continue;
-        const int z = plane[k];
-        const int lo = __builtin_amdgcn_readfirstlane(s.zs[max(z - NS + 1, 0)]);
-        const int hi = __builtin_amdgcn_readfirstlane(s.zs[min(z + 1, g.bin[2])]);
-        for (int i0 = lo; i0 < hi; i0 += 16) {
-          const int i = i0 + li;  // this lane's point
-          const bool in = i < hi;
-          const double kz = s.kz[i * kPitch + (z & 15)];
-          d4 re = {}, im = {};
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const double w = in ? s.ky[i * kPitch + 4 * q + lk] * kz : 0.0;
-            re = __builtin_amdgcn_mfma_f64_16x16x4f64(v[k][q].x, w, re, 0, 0, 0);
-            im = __builtin_amdgcn_mfma_f64_16x16x4f64(v[k][q].y, w, im, 0, 0, 0);
-          }
-          // lane holds cells x = 4 q + lk of its point: dot with kx, over lk
-          double sr = 0.0, si = 0.0;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const double w = s.kx[i * kPitch + 4 * q + lk];
-            sr = fma(w, re[q], sr);
-            si = fma(w, im[q], si);
-          }
-          sr += __shfl_xor(sr, 16, 64);
-          si += __shfl_xor(si, 16, 64);
-          sr += __shfl_xor(sr, 32, 64);
-          si += __shfl_xor(si, 32, 64);
-          if (lk == 0 && in) {
-            const Cplx<double> o = part[wave][i];
-            part[wave][i] = Cplx<double>{o.x + sr, o.y + si};
-          }
-        }
-        // later chunks reach the planes from zlast on, this one those below
-        // zlast + NS
-        open[k] = last ? z + 2 * kPlaneWaves < zlast + NS : z < zlast;
-        if (last || z < zlast) plane[k] = z + 2 * kPlaneWaves;
-        if (open[k]) load_plane(k);
-        open[k] = open[k] && plane[k] < ext[2];
+      for (int q = 0; q < 4; ++q) {
+        const int j = 4 * q + lk - r1;
+        const double w = ky[i * kP + min(max(j, 0), NS - 1)];
+        wy[q] = in && j >= 0 && j < NS ? w : 0.0;
       }
-    }
-    __syncthreads();
-    if (static_cast<int>(threadIdx.x) < cnt) {
+      d4 re = {}, im = {};
+      // a plane's cells are loaded behind the products of the plane before
+      Cplx<double> even[4], odd[4];
+      auto load = [&](int z, Cplx<double> (&v)[4]) __attribute__((always_inline)) {
+        const Cplx<double>* src = plane_at(z);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = src[row[q]];
+      };
+      auto add = [&](int z, const Cplx<double> (&v)[4]) __attribute__((always_inline)) {
+        const int j = z - r2;
+        double wz = kz[i * kP + min(max(j, 0), NS - 1)];
+        wz = j >= 0 && j < NS ? wz : 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const double w = wy[q] * wz;
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q].x, w, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(v[q].y, w, im, 0, 0, 0);
+        }
+      };
+      load(zbeg, even);
+      for (int z = zbeg; z < zend; z += 2) {
+        if (z + 1 < zend) load(z + 1, odd);
+        add(z, even);
+        if (z + 1 >= zend) break;
+        if (z + 2 < zend) load(z + 2, even);
+        add(z + 1, odd);
+      }
+      // lane holds cells x = 4 q + lk of its point: dot with kx, over lk
       double sr = 0.0, si = 0.0;
 #pragma unroll
-      for (int w = 0; w < kPlaneWaves; ++w) {
-        sr += part[w][threadIdx.x].x;
-        si += part[w][threadIdx.x].y;
+      for (int q = 0; q < 4; ++q) {
+        const int j = 4 * q + lk - r0;
+        double w = kx[i * kP + min(max(j, 0), NS - 1)];
+        w = j >= 0 && j < NS ? w : 0.0;
+        sr = fma(w, re[q], sr);
+        si = fma(w, im[q], si);
       }
-      const uint32_t p = sp.begin + base + threadIdx.x;
-      if (job.post) {
-        const Cplx<double> q = job.post[p];
-        const double tr = sr * q.x - si * q.y;
-        si = sr * q.y + si * q.x;
-        sr = tr;
+      sr += __shfl_xor(sr, 16, 64);
+      si += __shfl_xor(si, 16, 64);
+      sr += __shfl_xor(sr, 32, 64);
+      si += __shfl_xor(si, 32, 64);
+      const uint32_t dst = __shfl(to, i, 64);
+      if (lk == 0 && in) {
+        if (job.post) {
+          const Cplx<double> q = job.post[sp.begin + base + static_cast<uint32_t>(i)];
+          const double tr = sr * q.x - si * q.y;
+          si = sr * q.y + si * q.x;
+          sr = tr;
+        }
+        job.out[dst] = Cplx<double>{sr, si};
       }
-      job.out[job.perm[p]] = Cplx<double>{sr, si};
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
-// Workgroup b takes part b % split of subproblem b / split: `split` equal runs
-// of the largest subproblem's points; a run past the last point is empty.
+// Part `part` of a subproblem: near-equal runs of whole 16-point groups, at least
+// one group per wave; parts past the last point are empty. The launch takes all
+// first parts, then all second ones: empty parts between full ones leave every
+// other CU idle (128^3 cells, ns = 9, 0.02 points per cell: 66 us against 42).
 __device__ inline bool split_subproblem(Subprob& sp, uint32_t part, uint32_t split) {
-  const uint32_t run = kMaxSubproblemPoints / split;
+  const uint32_t run = max(16u * kInterpWaves, ((sp.count + split - 1) / split + 15u) & ~15u);
   if (part * run >= sp.count) return false;
   sp.begin += part * run;
   sp.count = min(run, sp.count - part * run);
@@ -371,29 +384,30 @@ __device__ inline bool split_subproblem(Subprob& sp, uint32_t part, uint32_t spl
 }
 
 template <int NS>
-__global__ void __launch_bounds__(kPlaneThreads, 4)
+__global__ void __launch_bounds__(kInterpThreads, 4)
     plane_interp_kernel(InterpJob<double, 3> job, const Subprob* __restrict__ subs, uint32_t nsub,
                         uint32_t split, EsParams es) {
-  const uint32_t b = xcd_remap(blockIdx.x, nsub * split);
-  Subprob sp = subs[b / split];
-  if (split_subproblem(sp, b % split, split)) plane_interp<NS>(job, sp, es);
+  Subprob sp = subs[xcd_remap(blockIdx.x % nsub, nsub)];
+  if (split_subproblem(sp, blockIdx.x / nsub, split)) plane_interp<NS>(job, sp, es);
 }
 
 template <int NS>
-__global__ void __launch_bounds__(kPlaneThreads, 4)
+__global__ void __launch_bounds__(kInterpThreads, 4)
     plane_interp_batch_kernel(const InterpJob<double, 3>* __restrict__ jobs,
                               const Subprob* __restrict__ subs, uint32_t nsub, uint32_t split,
                               EsParams es) {
-  const uint32_t b = xcd_remap(blockIdx.x, nsub * split);
-  Subprob sp = subs[b / split];
-  if (!split_subproblem(sp, b % split, split)) return;
+  Subprob sp = subs[xcd_remap(blockIdx.x % nsub, nsub)];
+  if (!split_subproblem(sp, blockIdx.x / nsub, split)) return;
   const InterpJob<double, 3> job = jobs[sp.job];
   plane_interp<NS>(job, sp, es);
 }
 
-// Two workgroups fit a CU, so fewer than 512 subproblems leave the chip idle;
-// each part reads the planes its own points touch.
-uint32_t interp_split(std::size_t nsub) { return nsub <= 512 ? 4u : (nsub <= 1024 ? 2u : 1u); }
+// Parts per subproblem: about 2048 workgroups of four waves fill the chip
+// (four on a CU) twice. 64^3 cells at 0.5 points per cell, ns = 9 (192
+// subproblems): 76 us in one part each, 50 in eight.
+uint32_t interp_split(std::size_t nsub) {
+  return static_cast<uint32_t>(std::min<std::size_t>(8, (2048 + nsub - 1) / nsub));
+}
 
 constexpr int kOrderThreads = 1024;
 constexpr int kOrderPerThread = static_cast<int>(kMaxSubproblemPoints) / kOrderThreads;
@@ -451,7 +465,7 @@ void interp_ns(const InterpJob<double, 3>& job, const Subprob* subs, std::size_t
                const EsParams& es, hipStream_t stream) {
   const uint32_t split = interp_split(nsub);
   hipLaunchKernelGGL((plane_interp_kernel<NS>), dim3(static_cast<unsigned>(nsub) * split),
-                     dim3(kPlaneThreads), 0, stream, job, subs,
+                     dim3(kInterpThreads), 0, stream, job, subs,
                      static_cast<uint32_t>(nsub), split, es);
   check_launch("plane_interp_kernel");
 }
@@ -461,7 +475,7 @@ void interp_batch_ns(const InterpJob<double, 3>* jobs, const Subprob* subs, std:
                      const EsParams& es, hipStream_t stream) {
   const uint32_t split = interp_split(nsub);
   hipLaunchKernelGGL((plane_interp_batch_kernel<NS>), dim3(static_cast<unsigned>(nsub) * split),
-                     dim3(kPlaneThreads), 0, stream, jobs, subs,
+                     dim3(kInterpThreads), 0, stream, jobs, subs,
                      static_cast<uint32_t>(nsub), split, es);
   check_launch("plane_interp_batch_kernel");
 }
