@@ -29,6 +29,7 @@
 // src/neonufft/gpu/kernels/spreading_kernel.cu:588-660,
 // interpolation_kernel.cu:193-319).
 #include <algorithm>
+#include <cfloat>
 
 #include "es_device.hpp"
 
@@ -350,6 +351,27 @@ __device__ __forceinline__ void plane_interp(const InterpJob<double, 3>& job, co
         w = j >= 0 && j < NS ? w : 0.0;
         sr = fma(w, re[q], sr);
         si = fma(w, im[q], si);
+      }
+      if (__any(!(fabs(sr) + fabs(si) <= DBL_MAX))) {
+        // An infinity or NaN in a cell times a zero weight is NaN for all 16
+        // points: each reads its own cells instead, lane lk the rows lk, lk + 4, ..
+        sr = si = 0.0;
+        for (int c = 0; in && c < NS; ++c) {
+          const Cplx<double>* src = plane_at(r2 + c);
+          for (int b = lk; b < NS; b += 4) {
+            const std::size_t line = static_cast<std::size_t>(g.n[0]) *
+                                     static_cast<std::size_t>(wrap_once(org[1] + r1 + b, g.n[1]));
+            double tr = 0.0, ti = 0.0;
+            for (int a = 0; a < NS; ++a) {
+              const Cplx<double> v = src[line + wrap_once(org[0] + r0 + a, g.n[0])];
+              tr = fma(kx[i * kP + a], v.x, tr);
+              ti = fma(kx[i * kP + a], v.y, ti);
+            }
+            const double w = ky[i * kP + b] * kz[i * kP + c];
+            sr = fma(w, tr, sr);
+            si = fma(w, ti, si);
+          }
+        }
       }
       sr += __shfl_xor(sr, 16, 64);
       si += __shfl_xor(si, 16, 64);
