@@ -200,7 +200,10 @@ std::pair<int, int> point_signature(const neonufft::Options& opt, IntType num_nu
                              static_cast<IntType>(static_cast<double>(modes[d]) * opt.upsampfac));
   }
   const int no_bin[3] = {0, 0, 0};
-  const BinGeom g = choose_bins(DIM, n, ks.ns, sizeof(Cplx<T>), no_bin);
+  double cells = 1.0;
+  for (int d = 0; d < DIM; ++d) cells *= static_cast<double>(n[d]);
+  const BinGeom g = choose_bins(DIM, n, ks.ns, sizeof(Cplx<T>), no_bin,
+                                plane_tiles_pay(ks.ns, static_cast<double>(num_nu), cells));
   Loc<T> l{{nullptr, nullptr, nullptr}};
   for (int d = 0; d < DIM; ++d) l.p[d] = loc[d];
   const FoldParams fp{{0, 0, 0}, {1, 1, 1}};

@@ -124,6 +124,12 @@ public:
       it.group = f->second;
       groups_[it.group].members.push_back(t);
     }
+    double points = 0.0, all_cells = 0.0;
+    for (int t = 0; t < count_; ++t) {
+      points += static_cast<double>(num_nu[t]);
+      all_cells += static_cast<double>(items_[t].n[0]) * static_cast<double>(items_[t].n[1]) *
+                   static_cast<double>(items_[t].n[2]);
+    }
     // lay the grids out group by group, each group starting on a 256-byte
     // boundary (the up/downsampling kernels store cell pairs as 16 bytes)
     std::size_t off = 0;
@@ -151,7 +157,9 @@ public:
         g.fs[d].reset(static_cast<std::size_t>(g.n[d] / 2 + 1), alloc_);
         launch_fseries<T>(g.fs[d].data(), g.n[d], ks_.quad, stream_);
       }
-      g.geom = choose_bins(DIM, g.n, ks_.ns, sizeof(Cplx<T>), tune_.bin);
+      // one launch spreads every group: the batch as a whole sets the density
+      g.geom = choose_bins(DIM, g.n, ks_.ns, sizeof(Cplx<T>), tune_.bin,
+                           plane_tiles_pay(ks_.ns, points, all_cells));
       g.cover.build(DIM, g.geom, ks_.ns, stream_, alloc_);
       max_lds_ = std::max(max_lds_, tile_bytes<T>(g.geom));
       max_n0_ = std::max(max_n0_, g.geom.n[0]);

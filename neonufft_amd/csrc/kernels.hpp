@@ -168,9 +168,11 @@ void launch_interp_batch(int ns, const InterpJob<T, DIM>* jobs, const Subprob* s
                          hipStream_t stream);
 
 // ---- planes.hip: 3D fp64 spreading / interpolation on the matrix cores ------
-// Tiles of at most 16 x 16 cells in x and y take it, kernels up to 12 cells
-// wide (a wider one leaves bins of four cells and fewer in a 16-cell tile).
+// Tiles of at most 16 x 16 cells in x and y take it, kernels 7 to 12 cells wide:
+// a wider one leaves bins of four cells and fewer in a 16-cell tile, narrower
+// ones are faster on LDS tiles (plane_tiles_pay in params.cpp).
 constexpr int kPlaneCells = 16;
+constexpr int kPlaneMinWidth = 7;
 constexpr int kPlaneMaxWidth = 12;
 constexpr int kMaxTilePlanes = 64;  // planes of one tile
 
@@ -178,7 +180,7 @@ constexpr int kMaxTilePlanes = 64;  // planes of one tile
 // spread / interpolated by the plane kernels.
 template <typename T, int DIM>
 bool plane_tiles(const BinGeom& g, int ns) {
-  return std::is_same_v<T, double> && DIM == 3 && ns <= kPlaneMaxWidth &&
+  return std::is_same_v<T, double> && DIM == 3 && ns >= kPlaneMinWidth && ns <= kPlaneMaxWidth &&
          g.tile[0] <= kPlaneCells && g.tile[1] <= kPlaneCells &&
          g.tile[2] <= kMaxTilePlanes;
 }

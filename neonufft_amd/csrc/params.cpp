@@ -168,6 +168,22 @@ int band_rows(IntType n0, IntType pitch, IntType n1, int ns, std::size_t acc_byt
   return rows >= 1 ? static_cast<int>(rows) : 0;
 }
 
+// Spreading on plane tiles is faster than on LDS tiles from ns = 7 on at any
+// density; interpolation from ns = 9 on, at ns = 8 below about one point per cell
+// and at ns = 7 below a third. A plan spreads and interpolates on the same
+// tiles. LDS tiles -> plane tiles, us of spreading | interpolation, 128^3 cells:
+//   ns = 7, 0.2 points per cell  188 -> 132 | 111 -> 99;   0.5  344 -> 273 | 179 -> 204
+//   ns = 8, 0.2                  310 -> 141 | 162 -> 123;  2   1756 -> 871 | 735 -> 765
+//   ns = 9, 0.2                  465 -> 160 | 223 -> 138;  2   2440 -> 1040 | 1038 -> 850
+// (worst: 64^3 cells, 1 point per cell, ns = 8: 126 -> 121 | 53 -> 74; ns = 9:
+// 171 -> 136 | 75 -> 81).
+// ns <= 6 gains at few points only (ns = 6, 0.05: 102 -> 63 | 69 -> 38; 0.5:
+// 248 -> 281 | 133 -> 190) and loses on small grids (ns = 5, 64^3 cells, 0.05:
+// 30 -> 39 | 15 -> 21), and clustered points are dense where they are.
+bool plane_tiles_pay(int ns, double points, double cells) {
+  return ns > kPlaneMinWidth || (ns == kPlaneMinWidth && 3.0 * points < cells);
+}
+
 BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
                     const int* bin_override, bool planes) {
   BinGeom g{};
@@ -196,7 +212,8 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
     }
   }
   int most[3] = {1 << 30, 1 << 30, 1 << 30};
-  if (dim == 3 && elem_bytes >= 16 && ns <= kPlaneMaxWidth && planes && !overridden) {
+  if (dim == 3 && elem_bytes >= 16 && ns >= kPlaneMinWidth && ns <= kPlaneMaxWidth && planes &&
+      !overridden) {
     // fp64 plane kernels: tiles of 16 x 16 cells
     most[0] = most[1] = pref[0] = pref[1] = kPlaneCells + 1 - ns;
     most[2] = kMaxTilePlanes + 1 - ns;

@@ -42,6 +42,10 @@ double fit_horner(int ns, double beta, int deg, double* coef /* ns*(deg+1) */);
 // in extended precision by Chebyshev interpolation.
 void fit_pairs(int ns, double beta, double* coef);
 
+// Whether 3D fp64 points on a grid of `cells` suit plane tiles (planes.hip) in
+// both directions.
+bool plane_tiles_pay(int ns, double points, double cells);
+
 // Bin geometry for a grid of size n (DIM entries), element size and ns.
 // bin_override: if non-null and positive entries, used instead of the default.
 // planes: 3D fp64 defaults suit the plane kernels (planes.hip).

@@ -176,7 +176,9 @@ public:
       fs_[d].reset(static_cast<std::size_t>(n_[d] / 2 + 1), alloc_);
       launch_fseries<T>(fs_[d].data(), n_[d], ks_.quad, stream_);
     }
-    geom_ = choose_bins(DIM, n_, ks_.ns, sizeof(Cplx<T>), tune_.bin);
+    geom_ = choose_bins(DIM, n_, ks_.ns, sizeof(Cplx<T>), tune_.bin,
+                        plane_tiles_pay(ks_.ns, static_cast<double>(num_nu),
+                                        static_cast<double>(cells)));
     cover_.build(DIM, geom_, ks_.ns, stream_, alloc_);
     if constexpr (DIM == 2) {
       band_ = plan_band_layout(n_, ks_.ns, sizeof(T), tune_, 256);
@@ -715,13 +717,14 @@ public:
       scale[d] = d < DIM ? gi_.gamma[d] * gi_.h[d] : 1.0;
       fp.scale[d] = scale[d];
     }
-    // Plane tiles of the outputs pay from about one point in ten cells: type 2
-    // fp64 at 0.22 points per cell 616 -> 460 us per pass, but 361 -> 417 us of
-    // interpolation at 0.024, where groups of 16 points are half empty.
-    std::size_t cells = 1;
-    for (int d = 0; d < DIM; ++d) cells *= static_cast<std::size_t>(gi_.fft_grid_size[d]);
-    const BinGeom geom = choose_bins(DIM, gi_.fft_grid_size, ks_.ns, sizeof(Cplx<T>), tune_.bin,
-                                     static_cast<std::size_t>(num_out) >= cells / 10);
+    // The targets fill 1 / upsampfac of each axis: those cells set the density.
+    double cells = 1.0;
+    for (int d = 0; d < DIM; ++d) {
+      cells *= static_cast<double>(gi_.fft_grid_size[d]) / opt_.upsampfac;
+    }
+    const BinGeom geom =
+        choose_bins(DIM, gi_.fft_grid_size, ks_.ns, sizeof(Cplx<T>), tune_.bin,
+                    plane_tiles_pay(ks_.ns, static_cast<double>(num_out), cells));
     out_pts_.build(l, static_cast<std::size_t>(num_out), fp, geom, ks_.ns, tune_.max_points,
                    stream_, alloc_);
     geom_out_ = geom;  // of the points held: a refused call keeps points and bins together
@@ -877,7 +880,9 @@ private:
       fs_[d].reset(static_cast<std::size_t>(gi_.fft_grid_size[d] / 2 + 1), alloc_);
       launch_fseries<T>(fs_[d].data(), gi_.fft_grid_size[d], ks_.quad, stream_);
     }
-    geom_in_ = choose_bins(DIM, gi_.spread_grid_size, ks_.ns, sizeof(Cplx<T>), tune_.bin);
+    // the inputs are only spread: plane tiles at any density from ns = 7 on
+    geom_in_ = choose_bins(DIM, gi_.spread_grid_size, ks_.ns, sizeof(Cplx<T>), tune_.bin,
+                           plane_tiles_pay(ks_.ns, 0.0, 1.0));
     cover_in_.build(DIM, geom_in_, ks_.ns, stream_, alloc_);
     check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
   }

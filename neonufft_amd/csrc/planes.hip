@@ -506,18 +506,13 @@ void interp_batch_ns(const InterpJob<double, 3>* jobs, const Subprob* subs, std:
 
 #define NNF_PLANE_CASES(FN, ...)                                       \
   switch (ns) {                                                        \
-    case 2: FN<2>(__VA_ARGS__); break;                                 \
-    case 3: FN<3>(__VA_ARGS__); break;                                 \
-    case 4: FN<4>(__VA_ARGS__); break;                                 \
-    case 5: FN<5>(__VA_ARGS__); break;                                 \
-    case 6: FN<6>(__VA_ARGS__); break;                                 \
     case 7: FN<7>(__VA_ARGS__); break;                                 \
     case 8: FN<8>(__VA_ARGS__); break;                                 \
     case 9: FN<9>(__VA_ARGS__); break;                                 \
     case 10: FN<10>(__VA_ARGS__); break;                               \
     case 11: FN<11>(__VA_ARGS__); break;                               \
     case 12: FN<12>(__VA_ARGS__); break;                               \
-    default: throw neonufft::InternalError("n_spread not in [2, 12]"); \
+    default: throw neonufft::InternalError("n_spread not in [7, 12]"); \
   }
 
 void launch_plane_spread(int ns, const SpreadJob<double, 3>& job, const Subprob* subs,
