@@ -212,12 +212,18 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
     }
   }
   int most[3] = {1 << 30, 1 << 30, 1 << 30};
-  if (dim == 3 && elem_bytes >= 16 && ns >= kPlaneMinWidth && ns <= kPlaneMaxWidth && planes &&
-      !overridden) {
-    // fp64 plane kernels: tiles of 16 x 16 cells
-    most[0] = most[1] = pref[0] = pref[1] = kPlaneCells + 1 - ns;
-    most[2] = kMaxTilePlanes + 1 - ns;
-    pref[2] = 32 + 1 - ns;
+  if (dim == 3 && elem_bytes >= 16 && ns >= kPlaneMinWidth && ns <= kPlaneMaxWidth) {
+    // fp64 plane kernels: tiles of 16 x 16 cells. Edges asked for that fit one
+    // are kept in one, so that a plan's own edges, passed back, give its tiles.
+    const int edge = kPlaneCells + 1 - ns, depth = kMaxTilePlanes + 1 - ns;
+    if (!overridden && planes) {
+      pref[0] = pref[1] = edge;
+      pref[2] = 32 + 1 - ns;
+    }
+    if (pref[0] <= edge && pref[1] <= edge && pref[2] <= depth) {
+      most[0] = most[1] = edge;
+      most[2] = depth;
+    }
   }
   // LDS tile bytes per workgroup (160 KB per CU on gfx950). Measured on MI355X
   // with 128^3 modes: fp64 tiles need most of it, since at ns >= 9 a 60 KB
@@ -239,36 +245,39 @@ BinGeom choose_bins(int dim, const IntType* n, int ns, std::size_t elem_bytes,
     if (pref[dmax] <= 1) break;
     pref[dmax] = std::max(1, pref[dmax] / 2);
   }
+  const int cap = dim == 3 ? CellPack<3>::max_bin : (dim == 2 ? CellPack<2>::max_bin : CellPack<1>::max_bin);
+  for (int d = 0; d < dim; ++d) pref[d] = std::max(1, std::min({pref[d], static_cast<int>(n[d]), cap}));
   // Prefer bin edges that leave no partial last bin narrower than ns - 1 (the tile
   // reduction then only needs a bin's direct neighbours): search the nearest
-  // edge within max(a quarter of the preferred one, ns) whose tile still fits.
-  for (int d = 0; d < dim; ++d) {
-    const int nd = static_cast<int>(n[d]);
-    const int B = std::min(pref[d], nd);
-    const auto good = [&](int b) { const int r = nd % b; return r == 0 || r >= ns - 1; };
-    if (B < ns - 1 || good(B)) continue;
-    const int span = std::max(B / 4, ns);
-    for (int delta = 1; delta <= span; ++delta) {
-      bool found = false;
-      for (int cand : {B - delta, B + delta}) {
-        if (cand < ns - 1 || cand > nd || cand > most[d]) continue;
-        int trial[3] = {pref[0], pref[1], pref[2]};
-        trial[d] = cand;
-        if (good(cand) && bytes(trial) <= budget) {
-          pref[d] = cand;
-          found = true;
-          break;
+  // edge within max(a quarter of the preferred one, ns) whose tile still fits,
+  // again while an edge moves (a smaller edge can make room for another).
+  for (bool moved = true; moved;) {
+    moved = false;
+    for (int d = 0; d < dim; ++d) {
+      const int nd = static_cast<int>(n[d]);
+      const int B = pref[d];
+      const auto good = [&](int b) { const int r = nd % b; return r == 0 || r >= ns - 1; };
+      if (B < ns - 1 || good(B)) continue;
+      const int span = std::max(B / 4, ns);
+      for (int delta = 1; delta <= span && pref[d] == B; ++delta) {
+        for (int cand : {B - delta, B + delta}) {
+          if (cand < ns - 1 || cand > nd || cand > cap || cand > most[d]) continue;
+          int trial[3] = {pref[0], pref[1], pref[2]};
+          trial[d] = cand;
+          if (good(cand) && bytes(trial) <= budget) {
+            pref[d] = cand;
+            moved = true;
+            break;
+          }
         }
       }
-      if (found) break;
     }
   }
   for (int d = 0; d < 3; ++d) {
     if (d < dim) {
       const int nd = static_cast<int>(n[d]);
-      const int cap = dim == 3 ? CellPack<3>::max_bin : (dim == 2 ? CellPack<2>::max_bin : CellPack<1>::max_bin);
       g.n[d] = nd;
-      g.bin[d] = std::max(1, std::min({pref[d], nd, cap}));
+      g.bin[d] = pref[d];
       g.nbins[d] = (nd + g.bin[d] - 1) / g.bin[d];
       g.tile[d] = g.bin[d] + ns - 1;
     } else {

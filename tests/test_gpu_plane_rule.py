@@ -81,3 +81,14 @@ def test_type3(tol, targets):
     # the kernel's own error: the requested tolerance, per axis and stage
     got = out.cpu().numpy()
     assert np.linalg.norm(got - ref) < 10 * tol * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("prec,tol,modes", [("f64", 1e-8, (96, 75, 80)), ("f64", 1e-6, (31, 64, 29)),
+                                            ("f32", 1e-5, (20, 33, 41)), ("f32", 1e-8, (9, 82, 9))])
+def test_reported_bins_give_the_same_plan(prec, tol, modes):
+    dt = torch.float64 if prec == "f64" else torch.float32
+    rng = np.random.default_rng(6)
+    dx = [dev(rng.uniform(-np.pi, np.pi, 3000), dt) for _ in range(3)]
+    opt = nnf.Options(tol=tol)
+    info = nnf.Plan(opt, -1, 3000, dx, modes).info()
+    assert nnf.Plan(opt, -1, 3000, dx, modes, bin_size=info["bin_size"]).info() == info
