@@ -141,7 +141,9 @@ struct Candidate {
   uint32_t max_points;
 };
 
-std::vector<Candidate> candidates(int dim) {
+// 3D fp64: the default tiles and the plane tiles too, whichever the default is
+// (no other candidate is narrow enough for the plane kernels).
+std::vector<Candidate> candidates(int dim, int ns, bool fp64) {
   std::vector<std::array<int, 3>> bins;
   if (dim == 1) {
     bins = {{1024, 1, 1}, {512, 1, 1}, {2048, 1, 1}, {256, 1, 1}};
@@ -150,6 +152,13 @@ std::vector<Candidate> candidates(int dim) {
   } else {
     bins = {{32, 8, 8}, {16, 16, 8}, {16, 8, 8}, {32, 16, 4}, {24, 8, 8}, {32, 8, 4},
             {64, 8, 4}, {16, 16, 4}};
+    if (fp64) {
+      bins.insert(bins.begin(), {0, 0, 0});
+      if (ns >= kPlaneMinWidth && ns <= kPlaneMaxWidth) {
+        const int edge = kPlaneCells + 1 - ns;
+        bins.push_back({edge, edge, 32 + 1 - ns});
+      }
+    }
   }
   std::vector<Candidate> out;
   for (uint32_t mp : {2048u, 1024u}) {
@@ -241,7 +250,8 @@ std::pair<nnf_tuning, double> tune(const neonufft::Options& opt, int sign, IntTy
   double best_ms = -1.0;
   std::vector<std::array<int64_t, 4>> seen;
   bool bands = false;  // type 1 spreads with row bands: tuned separately below
-  for (const Candidate& c : candidates(DIM)) {
+  const int ns = make_kernel_setup(opt.tol, opt.upsampfac, std::is_same_v<T, float>).ns;
+  for (const Candidate& c : candidates(DIM, ns, std::is_same_v<T, double>)) {
     PlanTuning t;
     for (int d = 0; d < 3; ++d) t.bin[d] = d < DIM ? c.bin[d] : 0;
     t.max_points = c.max_points;
