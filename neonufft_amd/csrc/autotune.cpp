@@ -18,8 +18,9 @@
 // disabled, in a text file that later processes read: NEONUFFT_AMD_TUNE_CACHE
 // names the file ("" disables it), else
 // $XDG_CACHE_HOME (or $HOME/.cache)/neonufft_amd/autotune-<version>-<gfx arch>.txt.
-// Every line of the file also carries the library version and the device's
-// architecture name, and only lines matching both are read.
+// Every line of the file also carries the library version with the kernels'
+// revision and the device's architecture name, and only lines matching both are
+// read.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,6 +48,10 @@ namespace {
 
 // precision, dim, ns, n0, n1, n2, log2 M, types, occupancy bucket, empty bucket
 using Key = std::tuple<int, int, int, int64_t, int64_t, int64_t, int, int, int, int>;
+
+// Version field of the cache lines. The revision goes up when kernels, default
+// tiles or candidates change: shapes tuned for others are timed again.
+const char* const kCacheVersion = NEONUFFT_VERSION "+r2";
 
 struct Entry {
   nnf_tuning tuning;
@@ -85,11 +90,11 @@ std::string cache_file(const std::string& arch) {
   return base + "/neonufft_amd/autotune-" + NEONUFFT_VERSION + "-" + arch + ".txt";
 }
 
-// One line per entry: "nnf-tune <version> <arch>" then the key fields, then
+// One line per entry: "nnf-tune <version>+r<revision> <arch>" then the key fields, then
 // bin_size[3] max_points spread_mode band_rows ms.
 std::string format_line(const std::string& arch, const Key& k, const nnf_tuning& t, double ms) {
   std::ostringstream o;
-  o << "nnf-tune " << NEONUFFT_VERSION << ' ' << arch << ' ' << std::get<0>(k) << ' '
+  o << "nnf-tune " << kCacheVersion << ' ' << arch << ' ' << std::get<0>(k) << ' '
     << std::get<1>(k) << ' ' << std::get<2>(k) << ' ' << std::get<3>(k) << ' ' << std::get<4>(k)
     << ' ' << std::get<5>(k) << ' ' << std::get<6>(k) << ' ' << std::get<7>(k) << ' '
     << std::get<8>(k) << ' ' << std::get<9>(k) << ' ' << t.bin_size[0] << ' ' << t.bin_size[1]
@@ -98,7 +103,7 @@ std::string format_line(const std::string& arch, const Key& k, const nnf_tuning&
   return o.str();
 }
 
-// Reads the file's entries for this version and architecture (once per file
+// Reads the file's entries for this version, revision and architecture (once per file
 // and process; a missing or unreadable file is an empty cache). Caller holds
 // g_cache_mutex.
 void load_file(const std::string& path, const std::string& arch) {
@@ -119,7 +124,7 @@ void load_file(const std::string& path, const std::string& arch) {
           t.spread_mode >> t.band_rows >> ms)) {
       continue;
     }
-    if (tag != "nnf-tune" || ver != NEONUFFT_VERSION || a != arch) continue;
+    if (tag != "nnf-tune" || ver != kCacheVersion || a != arch) continue;
     const Key k{prec, dim, ns, n0, n1, n2, mb, types, occ, empty};
     if (!g_cache.count(k)) g_cache[k] = Entry{t, ms, 2};
   }
