@@ -344,7 +344,8 @@ template <typename TC, int DIM>
 void launch_bin_count(Loc<TC> loc, std::size_t m, const FoldParams& fp, const BinGeom& g, int ns,
                       uint32_t* count, uint32_t* rank, uint32_t stride, hipStream_t stream) {
   if (m == 0) return;
-  if (m >= kLargeChunkMin) {
+  const std::size_t nbins = static_cast<std::size_t>(g.nbins[0]) * g.nbins[1] * g.nbins[2];
+  if (m >= kLargeChunkMin && m >= kLargeChunkPerBin * nbins) {
     constexpr int NT = kLargeChunkThreads;
     hipLaunchKernelGGL((bin_count_kernel<TC, DIM, NT>), dim3(chunk_rank_blocks(m, NT)), dim3(NT), 0,
                        stream, loc, m, fp, g, ns, count, rank, stride);
