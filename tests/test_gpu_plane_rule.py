@@ -92,3 +92,22 @@ def test_reported_bins_give_the_same_plan(prec, tol, modes):
     opt = nnf.Options(tol=tol)
     info = nnf.Plan(opt, -1, 3000, dx, modes).info()
     assert nnf.Plan(opt, -1, 3000, dx, modes, bin_size=info["bin_size"]).info() == info
+
+
+@pytest.mark.parametrize("modes,m", [((12, 12, 12), 40000), ((12, 12, 12), 70), ((40, 40, 40), 30000),
+                                     ((64, 64, 64), 30000), ((80, 72, 76), 20000)])
+def test_parts_of_subproblems(modes, m):
+    """Interpolation cuts subproblems into eight parts (few of them) down to one
+    (many); parts of one point, empty ones and full ones."""
+    rng = np.random.default_rng(m)
+    tol, n = 1e-8, int(np.prod(modes))
+    x, dx = _points(m, rng)
+    x[0][: m // 2] = rng.uniform(0.2, 0.25, m // 2)  # half of them in few bins
+    dx[0] = dev(x[0], torch.float64)
+    f = cplx(rng, n, "f64")
+    plan = nnf.Plan(nnf.Options(tol=tol), -1, m, dx, modes)
+    assert max(plan.info()["bin_size"][:2]) + plan.info()["n_spread"] - 1 <= 16
+    back = torch.zeros(m, dtype=torch.complex128, device="cuda")
+    plan.transform_type_2(dev(f, torch.complex128), None, back)
+    torch.cuda.synchronize()
+    assert O.rel_l2(back.cpu().numpy(), O.nufft2(x, f, modes, -1, tol)) < 1e-10
