@@ -163,10 +163,15 @@ __global__ void __launch_bounds__(kRowBlock)
   }
 }
 
-__global__ void clear_kernel(unsigned long long* __restrict__ p, std::size_t n) {
+__global__ void clear_kernel(unsigned long long* __restrict__ p, std::size_t n,
+                             uint32_t* __restrict__ ones, std::size_t num_ones) {
   for (std::size_t i = threadIdx.x + static_cast<std::size_t>(blockIdx.x) * blockDim.x; i < n;
        i += static_cast<std::size_t>(gridDim.x) * blockDim.x) {
     p[i] = 0ull;
+  }
+  for (std::size_t i = threadIdx.x + static_cast<std::size_t>(blockIdx.x) * blockDim.x; i < num_ones;
+       i += static_cast<std::size_t>(gridDim.x) * blockDim.x) {
+    ones[i] = 1u;
   }
 }
 
@@ -578,9 +583,11 @@ void launch_row_window_max(const uint32_t* bcount, int n1, int ns, uint32_t* out
   check_launch("row_window_max_kernel");
 }
 
-void launch_clear_bounds(unsigned long long* words, std::size_t n, hipStream_t stream) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(clear_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, words, n);
+void launch_clear_bounds(unsigned long long* words, std::size_t n, hipStream_t stream,
+                         uint32_t* ones, std::size_t num_ones) {
+  if (n == 0 && num_ones == 0) return;
+  hipLaunchKernelGGL(clear_kernel, dim3(blocks_for(std::max(n, num_ones), 256)), dim3(256), 0, stream,
+                     words, n, ones, num_ones);
   check_launch("clear_kernel");
 }
 

@@ -253,7 +253,9 @@ void launch_row_window_max(const uint32_t* bcount, int n1, int ns, uint32_t* out
 // Zeroes n 8-byte words of strength bounds (a kernel, so graphs may record
 // it). Each job owns band_bound_words(n1, sizeof(T)) words: its n1 row sums,
 // then its n1 row maxima.
-void launch_clear_bounds(unsigned long long* words, std::size_t n, hipStream_t stream);
+// (ones[0 .. num_ones) = 1 in the same launch)
+void launch_clear_bounds(unsigned long long* words, std::size_t n, hipStream_t stream,
+                         uint32_t* ones = nullptr, std::size_t num_ones = 0);
 inline std::size_t band_bound_words(int n1, std::size_t tbytes) {
   return (2 * static_cast<std::size_t>(n1) * tbytes + 7) / 8;
 }

@@ -375,14 +375,14 @@ public:
     if (!out || !out_strides) throw neonufft::InputError("Neonufft:: null output");
     if (pts_.size() && !in) throw neonufft::InputError("Neonufft:: null input");
     // Nothing refuses the call from here on. The grid is work memory again, and
-    // h is overwritten (the row kernels note it themselves).
+    // h is overwritten (noted by kernels that run anyway).
     T* fs[3] = {fs_[0].data(), fs_[1].data(), fs_[2].data()};
     if constexpr (DIM == 2) {
       if (bands_on_ && band_.fft) {
         // gather, then spread + x-FFT per band straight into the pruned
         // FFT's intermediate; y-FFT and deconvolution follow
-        grid_overwritten();
-        launch_clear_bounds(bounds_.data(), bounds_.size(), stream_);
+        launch_clear_bounds(bounds_.data(), bounds_.size(), stream_, formed_.data(), pencils_);
+        grid_partial_ = false;
         launch_band_gather<T>(nullptr, band_job(in), 1, pts_.size(), stream_);
         const int nb = static_cast<int>((n_[1] + band_rows_ - 1) / band_rows_);
         launch_band_spread<T>(ks_.ns, nullptr, nullptr, band_job(nullptr), 1,
